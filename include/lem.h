@@ -270,8 +270,8 @@ int lem_db_mask_loss(const float *E, const uint8_t *in_beam, int64_t K, double s
                      double ref_power, double eps, float *loss, float *grad_E, void *workspace,
                      int64_t workspace_bytes, void *stream);
 
-/* Batched-excitation contraction on FP32 MFMA: for F wavenumbers k_f and B = 64
- * excitation sets W at once,
+/* Batched-excitation contraction on MFMA (both factors split into three bfloat16
+ * parts, float32 sums): for F wavenumbers k_f and B = 64 excitation sets W at once,
  *   E[f,c,k,b] = sum_s G_c[k,s,f] W[f,s,b],
  *   G[k,s,f]   = F_f(r) (d . n_k) (e - d (d . e)),  F_f the lossy_propagation
  *                factor at wavenumber k_f (empropagation.py:768-801), e = (pol_x,
