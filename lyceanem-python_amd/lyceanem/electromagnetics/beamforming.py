@@ -9,7 +9,11 @@ numpy loop over command angles.  The weight builders and directivity_transform
 are host numpy restatements with the reference's arithmetic."""
 from __future__ import annotations
 
+import contextvars
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
+import torch
 
 from .. import _native
 
@@ -90,6 +94,34 @@ def directivity_transform(Etheta, Ephi, az_range=None, elev_range=None,
     return Ut / Uav, Up / Uav, Utot / Uav, Umax / Uav
 
 
+# Elements of one block of weight rows: the least that is worth a thread, and the
+# most whose float64 and complex128 temporaries stay in a core's cache.
+_BLOCK_MIN, _BLOCK_MAX = 1 << 14, 1 << 15
+
+
+def _in_row_blocks(work, n, width):
+    """work(slice) over the rows 0 .. n - 1 of `width` elements, a block at a time
+    in as many threads as torch uses on the host (numpy releases the interpreter
+    inside its operations): the same number of blocks for each.  The threads live
+    for this call and run in the caller's context (numpy's errstate).  Every
+    element is computed by the same numpy operations however the rows are cut.
+    2,701 commands x 256 elements: 73 ms in one piece, 9.5 in 16 threads;
+    1,891 x 81: 15.0, 4.4 (in 9; 5.8 in 16, which wait for each other too often)."""
+    threads = max(1, min(torch.get_num_threads(), n * width // _BLOCK_MIN))
+    rounds = -(-n * width // (threads * _BLOCK_MAX))
+    step = max(1, -(-n // max(threads * rounds, 1)))
+    blocks = [slice(i, min(i + step, n)) for i in range(0, n, step)]
+    threads = min(threads, len(blocks))
+    if threads < 2:
+        for b in blocks:
+            work(b)
+        return
+    with ThreadPoolExecutor(threads) as pool:
+        jobs = [pool.submit(contextvars.copy_context().run, work, b) for b in blocks]
+        for job in jobs:
+            job.result()
+
+
 def command_weights(Et, Ep, points, wavelength, az_range, elev_range, az_index, elev_index,
                     phase_resolution=24):
     """Weight rows of MaximumDirectivityMap, (n_az_index, n_elev_index, 3, ne)
@@ -102,24 +134,29 @@ def command_weights(Et, Ep, points, wavelength, az_range, elev_range, az_index, 
     ai = np.argmin(np.abs(np.asarray(az_range)[None, :] - cmd_az[:, None]), axis=1)
     ei = np.argmin(np.abs(np.asarray(elev_range)[None, :] - cmd_el[:, None]), axis=1)
     A, E = len(cmd_az), len(cmd_el)
-    W = np.empty((A, E, 3, ne), np.complex64)
-    # Et[:, ei, ai] for every (command az, command el)
-    W[:, :, 0] = np.exp(1j * -np.angle(Et[:, ei[None, :], ai[:, None]])).transpose(1, 2, 0)
-    W[:, :, 1] = np.exp(1j * -np.angle(Ep[:, ei[None, :], ai[:, None]])).transpose(1, 2, 0)
+    W = np.empty((A * E, 3, ne), np.complex64)
     # the reference's command angles are float32, so is its steering vector
     az_r = np.radians(cmd_az)[:, None]
     el_r = np.radians(cmd_el)[None, :]
     sv = np.stack(np.broadcast_arrays(*sph2cart(az_r, el_r, np.float32(1))), -1)
     sv = sv.reshape(-1, 3).astype(np.float64)
     p = np.asarray(points, np.float64).reshape(-1, 3)
-    for i in range(0, len(sv), 4096):
-        s = sv[i:i + 4096] * 1e9
+    row_el, row_az = np.tile(ei, A), np.repeat(ai, E)
+
+    def rows(r):
+        # Et[:, ei, ai] of the rows' commands
+        W[r, 0] = np.exp(1j * -np.angle(Et[:, row_el[r], row_az[r]])).T
+        W[r, 1] = np.exp(1j * -np.angle(Ep[:, row_el[r], row_az[r]])).T
+        s = sv[r] * 1e9
         dist = np.sqrt(np.abs((p[None, :, 0] - s[:, None, 0]) ** 2 +
                               (p[None, :, 1] - s[:, None, 1]) ** 2 +
                               (p[None, :, 2] - s[:, None, 2]) ** 2))
         dist = dist - dist.min(axis=1, keepdims=True)
         w = np.exp(1j * 2 * np.pi * (LIGHT_SPEED / wavelength) * (dist / LIGHT_SPEED))
-        W.reshape(-1, 3, ne)[i:i + 4096, 2] = w.astype(np.complex64)
+        W[r, 2] = w.astype(np.complex64)
+
+    _in_row_blocks(rows, A * E, ne)
+    W = W.reshape(A, E, 3, ne)
     if phase_resolution <= 12:
         W = WeightTruncation(W, phase_resolution).astype(np.complex64)
     a_idx, e_idx = np.meshgrid(np.arange(A), np.arange(E), indexing="ij")
