@@ -893,8 +893,8 @@ class TD:
                     "roofline": {"bound": "valu-fp64", "achieved": flops / (tp * 1e-3) / 1e12,
                                  "peak": PEAK_FP64 / 1e12, "unit": "TFLOP/s",
                                  "frac": flops / (tp * 1e-3) / PEAK_FP64, "traffic": None}}
-        return {"kernel": "placement: k_time_wake + k_time_bins + k_trace_keys + radix sort + "
-                          "k_trace_starts/hist/conv", "kernel_ms": rest, "extra": extra,
+        return {"kernel": "placement: k_time_wake + k_time_bins + k_place_count/groups/"
+                          "buckets/move/sums/merge + k_trace_conv", "kernel_ms": rest, "extra": extra,
                 "roofline": {"bound": "hbm", "achieved": place / (rest * 1e-3) / 1e9,
                              "peak": PEAK_HBM / 1e9, "unit": "GB/s",
                              "frac": place / (rest * 1e-3) / PEAK_HBM, "traffic": None,

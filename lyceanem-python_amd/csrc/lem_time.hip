@@ -19,11 +19,10 @@
 //                  division), summed per (source, sink) slot in path order --
 //                  no atomics, deterministic.  out[slot][n][c] float64.
 //   trace        : the same summed over every path (the source and sink sums
-//                  of time_domain.calculate_scattering), out[n][c]: a stable
-//                  radix sort of the paths by start sample, per-sample sums of
-//                  the amplitudes in path order, then the excitation
-//                  convolution -- O(V + N E) instead of the reference's V x E
-//                  atomic additions, and deterministic.
+//                  of time_domain.calculate_scattering), out[n][c]: the paths'
+//                  amplitudes summed per start sample in a fixed order, then
+//                  the excitation convolution -- O(V + N E) instead of the
+//                  reference's V x E atomic additions, and deterministic.
 #include "lem_device.h"
 #include "lem_internal.h"
 #include "../../include/lem.h"
@@ -189,28 +188,41 @@ LEM_DEV double dkey_inv(unsigned long long k)
     return __longlong_as_double((long long)u);
 }
 
-__global__ __launch_bounds__(TB) void k_time_wake(const double *__restrict__ arrival, int64_t V,
-                                                  unsigned long long *__restrict__ key)
+// Bound by the read: four loads in flight a thread, and one atomic minimum per 16
+// wavefronts (16.8 M arrivals: 51 us with one load and one per 4 -> 30).
+constexpr int WAKE_TB = 1024, WAKE_BLOCKS = 1024;
+__global__ __launch_bounds__(WAKE_TB) void k_time_wake(const double *__restrict__ arrival,
+                                                       int64_t V,
+                                                       unsigned long long *__restrict__ key)
 {
-    __shared__ unsigned long long s[TB];
+    __shared__ unsigned long long s[WAKE_TB / 64];
     unsigned long long m = dkey(1.0);
-    for (int64_t i = (int64_t)blockIdx.x * TB + threadIdx.x; i < V; i += (int64_t)gridDim.x * TB) {
-        const double a = arrival[i];
-        if (a == a) {  // NaN arrivals take no part
-            const unsigned long long k = dkey(a);
-            m = k < m ? k : m;
-        }
+    const int64_t stride = (int64_t)gridDim.x * WAKE_TB;
+    for (int64_t i = (int64_t)blockIdx.x * WAKE_TB + threadIdx.x; i < V; i += 4 * stride) {
+        double a[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            a[q] = i + q * stride < V ? arrival[i + q * stride] : 1.0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (a[q] == a[q]) {  // NaN arrivals take no part
+                const unsigned long long k = dkey(a[q]);
+                m = k < m ? k : m;
+            }
     }
-    s[threadIdx.x] = m;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const unsigned long long k = __shfl_xor(m, off);
+        m = k < m ? k : m;
+    }
+    if ((threadIdx.x & 63) == 0)
+        s[threadIdx.x >> 6] = m;
     __syncthreads();
-    for (int off = TB / 2; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off)
-            s[threadIdx.x] = s[threadIdx.x + off] < s[threadIdx.x] ? s[threadIdx.x + off]
-                                                                   : s[threadIdx.x];
-        __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < WAKE_TB / 64; ++w)
+            m = s[w] < m ? s[w] : m;
+        atomicMin(key, m);
     }
-    if (threadIdx.x == 0)
-        atomicMin(key, s[0]);
 }
 
 __global__ void k_time_wake_init(unsigned long long *__restrict__ key)
@@ -286,7 +298,385 @@ __global__ __launch_bounds__(TB) void k_time_map(
     o[2] = a2;
 }
 
-// Trace: sort keys (start sample clamped to [0, N]; N = never placed).
+// Trace, up to TRACE_PART_SAMPLES samples: the paths move once, in path order, to
+// the bucket of 2^sh samples they start in (k_place_count, _groups, _buckets,
+// _move), with their amplitudes, so that what follows reads memory in order;
+// each workgroup of k_place_sums then orders SUMS_CH paths of a bucket by sample
+// in LDS and sums them, and k_place_merge adds a bucket's chunks.  Chunks are cut
+// by position, orders are stable, sums have a fixed shape: deterministic.  Paths
+// that start past the trace's end are in no bucket.
+//
+// Bound by memory: 8 + 32 bytes of a path read and 26 written by the count and the
+// move, 26 read by the sums.  The radix sort of (sample, path) that longer traces
+// use reads 24-byte amplitudes one by one, a line each.  16.8 M paths, 65,536
+// samples: 794 -> 435 us (count 30, move 206 = 4.7 TB/s, sums 147, merge 15,
+// scans 13); 16 M paths of which 1 % start within 1,000 samples, one bucket:
+// 69 ms (one wavefront added the rest) -> 215 us.  Past TRACE_PART_SAMPLES a bucket's sums no longer fit beside its
+// paths in LDS.  Measured and left: chunks of 4,096 in the move (one workgroup a
+// CU, 242 us) and in the sums (205), buckets of 512 samples (move 190, sums 160,
+// merge 20).
+constexpr int PT = 1024;         // threads
+constexpr int PW = PT / 64;
+constexpr int MOVE_R = 2, SUMS_R = 2;  // paths of one thread
+constexpr int MOVE_CH = PT * MOVE_R, SUMS_CH = PT * SUMS_R;
+constexpr int PLACE_NB = 256;    // most buckets
+constexpr int PLACE_GROUP = 64;  // chunks whose counts one workgroup adds up
+constexpr int PLACE_SH_MIN = 8, PLACE_SH_MAX = 10;
+constexpr int PLACE_COLS = 3 << PLACE_SH_MAX >> 10;  // sums of one thread, at most
+static_assert(PT == 1024, "PLACE_COLS");
+constexpr int64_t TRACE_PART_SAMPLES = (int64_t)PLACE_NB << PLACE_SH_MAX;
+
+// bucket and sample in the bucket of a start sample; -1 past the end.  Samples
+// before the trace's start count as its first, as in the sort.
+LEM_DEV int place_sample(int64_t b, int64_t N) { return b >= N ? -1 : (b < 0 ? 0 : (int)b); }
+
+// rank[r]: how many earlier entries of this wavefront (rounds of 64 lanes) have the
+// same digit; cnt (the wavefront's own, zero before) ends up with the digit counts.
+template <int R>
+LEM_DEV void wave_ranks(const int (&digit)[R], int bits, volatile uint16_t *cnt, int (&rank)[R])
+{
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int d = digit[r];
+        unsigned long long m = __ballot(d >= 0);
+        for (int b = 0; b < bits; ++b) {
+            const bool on = (d >> b) & 1;
+            const unsigned long long v = __ballot(on);
+            m &= on ? v : ~v;
+        }
+        if (d >= 0) {
+            const int base = cnt[d];
+            rank[r] = base + __popcll(m & ((1ull << lane) - 1));
+            __builtin_amdgcn_wave_barrier();
+            if (m >> lane == 1)
+                cnt[d] = (uint16_t)(base + __popcll(m));
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// Exclusive sum over the workgroup; total: the sum of all.
+LEM_DEV int block_exclusive(int x, int *s_wave, int *total)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int y = x;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int z = __shfl_up(y, off);
+        y += lane >= off ? z : 0;
+    }
+    if (lane == 63)
+        s_wave[wave] = y;
+    __syncthreads();
+    int before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < PW; ++w) {
+        before += w < wave ? s_wave[w] : 0;
+        all += s_wave[w];
+    }
+    *total = all;
+    return before + y - x;
+}
+
+// Ranks of the workgroup's entries by digit (nd digits): place[r] = position in the
+// stable order; first (of digit threadIdx.x) and *total as counted.  cnt: PW x nd.
+template <int R>
+LEM_DEV int block_places(const int (&digit)[R], int nd, int bits, uint16_t *cnt, int *s_wave,
+                         int (&place)[R], int *total)
+{
+    const int wave = threadIdx.x >> 6;
+    for (int i = threadIdx.x; i < PW * nd; i += PT)
+        cnt[i] = 0;
+    __syncthreads();
+    wave_ranks(digit, bits, cnt + wave * nd, place);
+    __syncthreads();
+    int n = 0;
+    if ((int)threadIdx.x < nd)
+        for (int w = 0; w < PW; ++w)
+            n += cnt[w * nd + threadIdx.x];
+    const int first = block_exclusive(n, s_wave, total);
+    if ((int)threadIdx.x < nd) {
+        int at = first;
+        for (int w = 0; w < PW; ++w) {
+            const int c = cnt[w * nd + threadIdx.x];
+            cnt[w * nd + threadIdx.x] = (uint16_t)at;  // at < 64 R PW where c > 0
+            at += c;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        if (digit[r] >= 0)
+            place[r] += cnt[wave * nd + digit[r]];
+    return first;
+}
+
+// entry r of this thread: the chunk in rounds of 64 lanes, wavefront by wavefront
+template <int R>
+LEM_DEV int place_entry(int r)
+{
+    return (threadIdx.x >> 6) * (64 * R) + r * 64 + (threadIdx.x & 63);
+}
+
+// counts[chunk][bucket]
+__global__ __launch_bounds__(PT) void k_place_count(const int64_t *__restrict__ bin, int64_t V,
+                                                    int64_t N, int sh, int *__restrict__ counts)
+{
+    __shared__ int s_n[PLACE_NB];
+    if (threadIdx.x < PLACE_NB)
+        s_n[threadIdx.x] = 0;
+    __syncthreads();
+    const int64_t c0 = (int64_t)blockIdx.x * MOVE_CH;
+#pragma unroll
+    for (int r = 0; r < MOVE_R; ++r) {
+        const int64_t v = c0 + r * PT + threadIdx.x;
+        const int k = v < V ? place_sample(bin[v], N) : -1;
+        if (k >= 0)
+            atomicAdd(&s_n[k >> sh], 1);
+    }
+    __syncthreads();
+    if (threadIdx.x < PLACE_NB)
+        counts[(int64_t)blockIdx.x * PLACE_NB + threadIdx.x] = s_n[threadIdx.x];
+}
+
+// counts -> the paths of the bucket in earlier chunks of the group; sums[group][bucket]
+__global__ __launch_bounds__(PLACE_NB) void k_place_groups(int *__restrict__ counts,
+                                                           int64_t nchunk, int *__restrict__ sums)
+{
+    const int64_t c0 = (int64_t)blockIdx.x * PLACE_GROUP;
+    const int64_t c1 = c0 + PLACE_GROUP < nchunk ? c0 + PLACE_GROUP : nchunk;
+    int at = 0;
+#pragma unroll 8
+    for (int64_t c = c0; c < c1; ++c) {
+        const int n = counts[c * PLACE_NB + threadIdx.x];
+        counts[c * PLACE_NB + threadIdx.x] = at;
+        at += n;
+    }
+    sums[(int64_t)blockIdx.x * PLACE_NB + threadIdx.x] = at;
+}
+
+// sums -> the bucket's first position plus its paths in earlier groups.
+// first[b]: bucket b's first position, chunk[b]: chunks of buckets before b.
+__global__ __launch_bounds__(PT) void k_place_buckets(int *__restrict__ sums, int64_t ngroup,
+                                                      int *__restrict__ first,
+                                                      int *__restrict__ chunk)
+{
+    __shared__ int s_part[PW * 64], s_wave[PW];
+    // PLACE_Q threads a bucket, each a share of the groups
+    const int b = threadIdx.x & (PLACE_NB - 1), q = threadIdx.x / PLACE_NB;
+    constexpr int PLACE_Q = PT / PLACE_NB;
+    const int64_t g0 = ngroup * q / PLACE_Q, g1 = ngroup * (q + 1) / PLACE_Q;
+    int n = 0;
+#pragma unroll 4
+    for (int64_t g = g0; g < g1; ++g)
+        n += sums[g * PLACE_NB + b];
+    s_part[q * PLACE_NB + b] = n;
+    __syncthreads();
+    int all = 0, before = 0;
+    for (int i = 0; i < PLACE_Q; ++i) {
+        all += s_part[i * PLACE_NB + b];
+        before += i < q ? s_part[i * PLACE_NB + b] : 0;
+    }
+    int total, chunks;
+    const int f = block_exclusive(q == 0 ? all : 0, s_wave, &total);
+    __syncthreads();
+    const int c = block_exclusive(q == 0 ? (int)(((int64_t)all + SUMS_CH - 1) / SUMS_CH) : 0,
+                                  s_wave, &chunks);
+    __syncthreads();
+    if (q == 0) {
+        s_part[b] = f;
+        first[b] = f;
+        chunk[b] = c;
+        if (b == 0) {
+            first[PLACE_NB] = total;
+            chunk[PLACE_NB] = chunks;
+        }
+    }
+    __syncthreads();
+    int at = s_part[b] + before;
+#pragma unroll 4
+    for (int64_t g = g0; g < g1; ++g) {
+        const int k = sums[g * PLACE_NB + b];
+        sums[g * PLACE_NB + b] = at;
+        at += k;
+    }
+}
+
+constexpr int PLACE_MOVE_LDS = MOVE_CH * (24 + 2 + 2) + PW * PLACE_NB * 2 + PLACE_NB * 4 + PW * 4;
+
+__global__ __launch_bounds__(PT) void k_place_move(
+    const int64_t *__restrict__ bin, const double *__restrict__ amp, int64_t V, int64_t N, int sh,
+    const int *__restrict__ counts, const int *__restrict__ sums, uint16_t *__restrict__ key,
+    double *__restrict__ moved)
+{
+    extern __shared__ __align__(16) char s_mem[];
+    double *s_amp = reinterpret_cast<double *>(s_mem);
+    uint16_t *s_key = reinterpret_cast<uint16_t *>(s_mem + MOVE_CH * 24);
+    uint16_t *s_bucket = s_key + MOVE_CH;
+    uint16_t *s_cnt = s_bucket + MOVE_CH;
+    int *s_to = reinterpret_cast<int *>(s_cnt + PW * PLACE_NB);
+    int *s_wave = s_to + PLACE_NB;
+    // an XCD takes consecutive chunks: the runs that share a line share its L2
+    const int64_t nchunk = (V + MOVE_CH - 1) / MOVE_CH;
+    const int64_t chunk = (blockIdx.x & 7) * ((nchunk + 7) / 8) + (blockIdx.x >> 3);
+    if (chunk >= nchunk)
+        return;
+    const int64_t c0 = chunk * MOVE_CH;
+    int digit[MOVE_R], local[MOVE_R], place[MOVE_R];
+    double a[MOVE_R][3];
+#pragma unroll
+    for (int r = 0; r < MOVE_R; ++r) {
+        const int64_t v = c0 + place_entry<MOVE_R>(r);
+        const int k = v < V ? place_sample(bin[v], N) : -1;
+        digit[r] = k >> sh;  // -1 stays -1
+        local[r] = k & ((1 << sh) - 1);
+    }
+#pragma unroll
+    for (int r = 0; r < MOVE_R; ++r)
+        if (digit[r] >= 0) {
+            const int64_t v = c0 + place_entry<MOVE_R>(r);
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                a[r][c] = amp[3 * v + c];
+        }
+    int n;
+    const int f = block_places(digit, PLACE_NB, 8, s_cnt, s_wave, place, &n);
+    if (threadIdx.x < PLACE_NB)
+        s_to[threadIdx.x] = counts[chunk * PLACE_NB + threadIdx.x] +
+                            sums[(chunk / PLACE_GROUP) * PLACE_NB + threadIdx.x] - f;
+#pragma unroll
+    for (int r = 0; r < MOVE_R; ++r)
+        if (digit[r] >= 0) {
+            s_key[place[r]] = (uint16_t)local[r];
+            s_bucket[place[r]] = (uint16_t)digit[r];
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                s_amp[3 * place[r] + c] = a[r][c];
+        }
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += PT)
+        key[(int64_t)s_to[s_bucket[i]] + i] = s_key[i];
+    for (int i = threadIdx.x; i < 3 * n; i += PT) {
+        const int p = i / 3;
+        moved[((int64_t)s_to[s_bucket[p]] + p) * 3 + (i - 3 * p)] = s_amp[i];
+    }
+}
+
+inline int place_sums_lds(int sh) { return SUMS_CH * 24 + ((PW * 2) << sh) + (1 << sh) * 2 + 8 + PW * 4; }
+
+// Sums of one chunk: part[chunk][sample of the bucket][3].  DIRECT: the trace is one
+// bucket, nothing was moved (key: none), and a workgroup adds up `per` chunks in
+// path order.
+template <bool DIRECT>
+__global__ __launch_bounds__(PT) void k_place_sums(
+    const int64_t *__restrict__ bin, const uint16_t *__restrict__ key,
+    const double *__restrict__ amp, int64_t V, int64_t N, int sh, const int *__restrict__ first,
+    const int *__restrict__ chunk, int64_t per, double *__restrict__ part)
+{
+    extern __shared__ __align__(16) char s_mem[];
+    double *s_amp = reinterpret_cast<double *>(s_mem);
+    const int nd = 1 << sh, cols = 3 * nd;
+    uint16_t *s_cnt = reinterpret_cast<uint16_t *>(s_mem + SUMS_CH * 24);
+    uint16_t *s_first = s_cnt + PW * nd;  // nd + 1 of them
+    int *s_wave = reinterpret_cast<int *>(s_first + nd + 2);
+    int64_t v0, v1;
+    if (DIRECT) {
+        v0 = (int64_t)blockIdx.x * per * SUMS_CH;
+        v1 = v0 + per * SUMS_CH < V ? v0 + per * SUMS_CH : V;
+    } else {
+        if ((int)blockIdx.x >= chunk[PLACE_NB])
+            return;
+        int lo = 0, hi = PLACE_NB;  // last bucket with chunk[b] <= id (buckets may be empty)
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (chunk[mid] <= (int)blockIdx.x)
+                lo = mid;
+            else
+                hi = mid;
+        }
+        v0 = (int64_t)first[lo] + (int64_t)((int)blockIdx.x - chunk[lo]) * SUMS_CH;
+        v1 = first[lo + 1];
+    }
+    double sum[PLACE_COLS] = {};
+    do {
+        int digit[SUMS_R], place[SUMS_R];
+        double a[SUMS_R][3];
+#pragma unroll
+        for (int r = 0; r < SUMS_R; ++r) {
+            const int64_t v = v0 + place_entry<SUMS_R>(r);
+            digit[r] = -1;
+            if (v < v1)
+                digit[r] = DIRECT ? place_sample(bin[v], N) : (int)key[v];
+            if (digit[r] >= 0) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c)
+                    a[r][c] = amp[3 * v + c];
+            }
+        }
+        int n;
+        const int f = block_places(digit, nd, sh, s_cnt, s_wave, place, &n);
+        if ((int)threadIdx.x < nd)
+            s_first[threadIdx.x] = (uint16_t)f;
+        if (threadIdx.x == 0)
+            s_first[nd] = (uint16_t)n;
+#pragma unroll
+        for (int r = 0; r < SUMS_R; ++r)
+            if (digit[r] >= 0)
+#pragma unroll
+                for (int c = 0; c < 3; ++c)
+                    s_amp[3 * place[r] + c] = a[r][c];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < PLACE_COLS; ++q) {
+            const int i = q * PT + threadIdx.x;
+            if (i >= cols)
+                break;
+            const int d = i / 3, c = i - 3 * d;
+            const int e = s_first[d + 1];
+            for (int p = s_first[d]; p < e; ++p)
+                sum[q] += s_amp[3 * p + c];
+        }
+        if (!DIRECT)
+            break;
+        v0 += SUMS_CH;
+        __syncthreads();
+    } while (v0 < v1);
+    double *out = part + (int64_t)blockIdx.x * cols;
+#pragma unroll
+    for (int q = 0; q < PLACE_COLS; ++q)
+        if (q * PT + (int)threadIdx.x < cols)
+            out[q * PT + threadIdx.x] = sum[q];
+}
+
+// H of a bucket: its chunks' sums, 16 strided shares and then those in order.
+// Grid: (ceil(3 * 2^sh / 64), buckets).
+__global__ __launch_bounds__(PT) void k_place_merge(const double *__restrict__ part,
+                                                    const int *__restrict__ chunk, int64_t direct,
+                                                    int64_t N, int sh, double *__restrict__ H)
+{
+    __shared__ double s[PW][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int cols = 3 << sh, col = blockIdx.x * 64 + lane, b = blockIdx.y;
+    const int64_t c0 = chunk ? chunk[b] : 0, c1 = chunk ? chunk[b + 1] : direct;
+    double h = 0.0;
+    if (col < cols) {
+#pragma unroll 4
+        for (int64_t c = c0 + wave; c < c1; c += PW)
+            h += part[c * cols + col];
+    }
+    s[wave][lane] = h;
+    __syncthreads();
+    const int64_t at = (int64_t)b * cols + col;
+    if (wave == 0 && col < cols && at < 3 * N) {
+#pragma unroll
+        for (int w = 1; w < PW; ++w)
+            h += s[w][lane];
+        H[at] = h;
+    }
+}
+
+// Longer traces: sort keys (start sample clamped to [0, N]; N = never placed).
 __global__ __launch_bounds__(TB) void k_trace_keys(const int64_t *__restrict__ bin, int64_t V,
                                                    int64_t N, int32_t *__restrict__ key,
                                                    int32_t *__restrict__ val)
@@ -294,11 +684,9 @@ __global__ __launch_bounds__(TB) void k_trace_keys(const int64_t *__restrict__ b
     const int64_t p = (int64_t)blockIdx.x * TB + threadIdx.x;
     if (p >= V)
         return;
-    // keys 0 .. N - 1 (a 2^16-sample trace sorts on 16 bits); a path that
-    // starts at or past the trace's end keeps key N - 1 and is marked -1
     const int64_t b = bin[p];
-    key[p] = (int32_t)(b < 0 ? 0 : (b >= N ? N - 1 : b));
-    val[p] = b >= N ? -1 : (int32_t)p;
+    key[p] = (int32_t)(b < 0 ? 0 : (b >= N ? N : b));
+    val[p] = (int32_t)p;
 }
 
 // start[b] = first sorted position with key >= b, for b in [0, N]
@@ -336,8 +724,6 @@ __global__ __launch_bounds__(TB) void k_trace_hist(const double *__restrict__ am
     const int32_t e = start[b + 1];
     for (int32_t i = start[b] + lane; i < e; i += 64) {
         const int64_t p = val[i];
-        if (p < 0)
-            continue;  // past the trace's end
         h0 += amp[3 * p];
         h1 += amp[3 * p + 1];
         h2 += amp[3 * p + 2];
@@ -355,31 +741,51 @@ __global__ __launch_bounds__(TB) void k_trace_hist(const double *__restrict__ am
     }
 }
 
-// out[n] = sum_{j <= min(E - 1, n)} exc[j] H[n - j]
-__global__ __launch_bounds__(TB) void k_trace_conv(const double *__restrict__ H,
+// out[n] = sum_{j <= min(E - 1, n)} exc[j] H[n - j]: 64 samples a workgroup, its 16
+// wavefronts take a share of the excitation each and the shares are added in order
+// (one wavefront a SIMD with all of it, 65,536 samples and 256 of excitation: 36 us;
+// this: 18).
+__global__ __launch_bounds__(PT) void k_trace_conv(const double *__restrict__ H,
                                                    const double *__restrict__ exc, int64_t E,
                                                    int64_t N, double *__restrict__ out)
 {
-    const int64_t n = (int64_t)blockIdx.x * TB + threadIdx.x;
-    if (n >= N)
-        return;
-    const int64_t J = n + 1 < E ? n + 1 : E;
+    __shared__ double s[PW][3][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t n = (int64_t)blockIdx.x * 64 + lane;
+    const int64_t share = (E + PW - 1) / PW;
+    const int64_t j0 = wave * share;
+    int64_t j1 = j0 + share < E ? j0 + share : E;
+    j1 = n < N ? (j1 < n + 1 ? j1 : n + 1) : 0;
     double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-    for (int64_t j = 0; j < J; ++j) {
+#pragma unroll 4
+    for (int64_t j = j0; j < j1; ++j) {
         const double e = exc[j];
         const double *h = H + 3 * (n - j);
         a0 += e * h[0];
         a1 += e * h[1];
         a2 += e * h[2];
     }
-    out[3 * n] = a0;
-    out[3 * n + 1] = a1;
-    out[3 * n + 2] = a2;
+    s[wave][0][lane] = a0;
+    s[wave][1][lane] = a1;
+    s[wave][2][lane] = a2;
+    __syncthreads();
+    if (threadIdx.x < 192) {
+        const int64_t at = (int64_t)blockIdx.x * 192 + threadIdx.x;
+        const int i = threadIdx.x / 3, c = threadIdx.x - 3 * i;
+        double a = 0.0;
+#pragma unroll
+        for (int w = 0; w < PW; ++w)
+            a += s[w][c][i];
+        if (at < 3 * N)
+            out[at] = a;
+    }
 }
 
 struct TraceWs {
     int32_t *k0, *k1, *v0, *v1, *start;
-    double *H;
+    int *counts, *sums, *first, *chunk;
+    uint16_t *key;
+    double *moved, *part, *H;
     void *cub;
     size_t cub_bytes;
 };
@@ -394,6 +800,21 @@ inline int key_bits(int64_t N)
 
 inline int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
 
+// log2 of a bucket's samples: as few as cover the trace, which keeps the chunks' sums
+// short; a trace of at most 2^PLACE_SH_MAX samples is one bucket and nothing moves.
+inline int place_shift(int64_t N)
+{
+    int sh = PLACE_SH_MIN;
+    while (sh < PLACE_SH_MAX && ((int64_t)PLACE_NB << sh) < N)
+        ++sh;
+    while (N <= ((int64_t)1 << PLACE_SH_MAX) && ((int64_t)1 << sh) < N)
+        ++sh;
+    return sh;
+}
+
+// Workgroups of k_place_sums<true>: four a CU or as many as there are chunks.
+inline int64_t place_direct(int64_t V) { return std::min<int64_t>(ceil_div(V, SUMS_CH), 1024); }
+
 // Lays the trace workspace out from base (or only sizes it when base is null).
 inline int64_t trace_layout(int64_t V, int64_t N, size_t cub_bytes, char *base, TraceWs *L)
 {
@@ -403,20 +824,33 @@ inline int64_t trace_layout(int64_t V, int64_t N, size_t cub_bytes, char *base, 
         off += align256(bytes);
         return p;
     };
-    char *k0 = take(4 * V), *k1 = take(4 * V), *v0 = take(4 * V), *v1 = take(4 * V);
-    char *st = take(4 * (N + 2));
-    char *H = take(8 * 3 * N);
-    char *cub = take((int64_t)cub_bytes);
-    if (L) {
-        L->k0 = reinterpret_cast<int32_t *>(k0);
-        L->k1 = reinterpret_cast<int32_t *>(k1);
-        L->v0 = reinterpret_cast<int32_t *>(v0);
-        L->v1 = reinterpret_cast<int32_t *>(v1);
-        L->start = reinterpret_cast<int32_t *>(st);
-        L->H = reinterpret_cast<double *>(H);
-        L->cub = cub;
-        L->cub_bytes = cub_bytes;
+    TraceWs l = {};
+    l.H = reinterpret_cast<double *>(take(8 * 3 * N));
+    if (N <= TRACE_PART_SAMPLES) {
+        const int sh = place_shift(N);
+        const int64_t nchunk = ceil_div(V, MOVE_CH);
+        const bool direct = N <= ((int64_t)1 << sh);
+        l.part = reinterpret_cast<double *>(
+            take((direct ? place_direct(V) : ceil_div(V, SUMS_CH) + PLACE_NB) * (24LL << sh)));
+        if (!direct) {
+            l.counts = reinterpret_cast<int *>(take(4 * PLACE_NB * nchunk));
+            l.sums = reinterpret_cast<int *>(take(4 * PLACE_NB * ceil_div(nchunk, PLACE_GROUP)));
+            l.first = reinterpret_cast<int *>(take(4 * (PLACE_NB + 1)));
+            l.chunk = reinterpret_cast<int *>(take(4 * (PLACE_NB + 1)));
+            l.key = reinterpret_cast<uint16_t *>(take(2 * V));
+            l.moved = reinterpret_cast<double *>(take(24 * V));
+        }
+    } else {
+        l.k0 = reinterpret_cast<int32_t *>(take(4 * V));
+        l.k1 = reinterpret_cast<int32_t *>(take(4 * V));
+        l.v0 = reinterpret_cast<int32_t *>(take(4 * V));
+        l.v1 = reinterpret_cast<int32_t *>(take(4 * V));
+        l.start = reinterpret_cast<int32_t *>(take(4 * (N + 2)));
+        l.cub = take((int64_t)cub_bytes);
+        l.cub_bytes = cub_bytes;
     }
+    if (L)
+        *L = l;
     return off;
 }
 
@@ -427,7 +861,7 @@ inline int64_t cub_sort_bytes(int64_t V, int64_t N)
     if (hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, (const int32_t *)nullptr,
                                            (int32_t *)nullptr, (const int32_t *)nullptr,
                                            (int32_t *)nullptr, (int)V, 0,
-                                           key_bits(N - 1)) != hipSuccess)
+                                           key_bits(N)) != hipSuccess)
         return -1;
     return (int64_t)bytes;
 }
@@ -462,8 +896,8 @@ extern "C" int lem_time_wake(const double *arrival, int64_t V, double *wake, voi
     unsigned long long *key = reinterpret_cast<unsigned long long *>(wake);
     hipLaunchKernelGGL(k_time_wake_init, dim3(1), dim3(64), 0, st, key);
     if (V > 0) {
-        const int64_t nb = std::min<int64_t>(ceil_div(V, TB), 1024);
-        hipLaunchKernelGGL(k_time_wake, dim3((unsigned)nb), dim3(TB), 0, st, arrival, V, key);
+        const int64_t nb = std::min<int64_t>(ceil_div(V, WAKE_TB), WAKE_BLOCKS);
+        hipLaunchKernelGGL(k_time_wake, dim3((unsigned)nb), dim3(WAKE_TB), 0, st, arrival, V, key);
     }
     hipLaunchKernelGGL(k_time_wake_finish, dim3(1), dim3(64), 0, st, key);
     return check_launch("k_time_wake");
@@ -510,10 +944,10 @@ extern "C" int64_t lem_time_trace_workspace(int64_t V, int64_t N)
 {
     if (V < 0 || N < 0 || V > 2000000000LL || N > 2000000000LL)
         return -1;
-    const int64_t cub = cub_sort_bytes(V > 0 ? V : 1, N);
+    const int64_t cub = N > TRACE_PART_SAMPLES ? cub_sort_bytes(V > 0 ? V : 1, N) : 0;
     if (cub < 0)
         return -1;
-    return trace_layout(V, N, (size_t)cub, nullptr, nullptr);
+    return trace_layout(V > 0 ? V : 1, N, (size_t)cub, nullptr, nullptr);
 }
 
 extern "C" int lem_time_trace(const double *amp, const int64_t *bin, int64_t V,
@@ -527,8 +961,9 @@ extern "C" int lem_time_trace(const double *amp, const int64_t *bin, int64_t V,
         return 0;
     LEM_REQUIRE(out && (V == 0 || (amp && bin)) && (E == 0 || excitation),
                 "lem_time_trace: null pointer");
+    LEM_REQUIRE(ceil_div(N, TB / 64) <= 2147483647LL, "lem_time_trace: too many samples");
     const int64_t Vs = V > 0 ? V : 1;
-    const int64_t cub = cub_sort_bytes(Vs, N);
+    const int64_t cub = N > TRACE_PART_SAMPLES ? cub_sort_bytes(Vs, N) : 0;
     if (cub < 0) {
         set_error("lem_time_trace: radix sort size query failed");
         return E_HIP;
@@ -542,25 +977,60 @@ extern "C" int lem_time_trace(const double *amp, const int64_t *bin, int64_t V,
     TraceWs L;
     trace_layout(Vs, N, cub_bytes, reinterpret_cast<char *>(workspace), &L);
     hipStream_t st = as_stream(stream);
-    if (V > 0) {
-        hipLaunchKernelGGL(k_trace_keys, dim3((unsigned)ceil_div(V, TB)), dim3(TB), 0, st, bin, V,
-                           N, L.k0, L.v0);
-        int rc = check_launch("k_trace_keys");
-        if (rc)
-            return rc;
-        size_t tb = L.cub_bytes;
-        if (hipcub::DeviceRadixSort::SortPairs(L.cub, tb, L.k0, L.k1, L.v0, L.v1, (int)V, 0,
-                                               key_bits(N - 1), st) != hipSuccess) {
-            set_error("lem_time_trace: radix sort failed");
-            return E_HIP;
+    int rc = 0;
+    if (N <= TRACE_PART_SAMPLES) {
+        const int sh = place_shift(N);
+        const int64_t nchunk = ceil_div(V, MOVE_CH), ngroup = ceil_div(nchunk, PLACE_GROUP);
+        const int64_t nsum = ceil_div(V, SUMS_CH);
+        const bool direct = N <= ((int64_t)1 << sh);
+        if (nchunk > 0 && direct) {
+            hipLaunchKernelGGL(k_place_sums<true>, dim3((unsigned)place_direct(V)), dim3(PT),
+                               place_sums_lds(sh), st, bin, nullptr, amp, V, N, sh, nullptr,
+                               nullptr, ceil_div(nsum, place_direct(V)), L.part);
+        } else if (!direct) {
+            if (nchunk > 0) {
+                hipLaunchKernelGGL(k_place_count, dim3((unsigned)nchunk), dim3(PT), 0, st, bin, V,
+                                   N, sh, L.counts);
+                hipLaunchKernelGGL(k_place_groups, dim3((unsigned)ngroup), dim3(PLACE_NB), 0, st,
+                                   L.counts, nchunk, L.sums);
+            }
+            hipLaunchKernelGGL(k_place_buckets, dim3(1), dim3(PT), 0, st, L.sums, ngroup, L.first,
+                               L.chunk);
+            if (nchunk > 0) {
+                hipLaunchKernelGGL(k_place_move, dim3((unsigned)(8 * ceil_div(nchunk, 8))), dim3(PT), PLACE_MOVE_LDS,
+                                   st, bin, amp, V, N, sh, L.counts, L.sums, L.key, L.moved);
+                hipLaunchKernelGGL(k_place_sums<false>, dim3((unsigned)(nsum + PLACE_NB)),
+                                   dim3(PT), place_sums_lds(sh), st, nullptr, L.key, L.moved, V, N,
+                                   sh, L.first, L.chunk, 1, L.part);
+            }
         }
+        const dim3 mg((unsigned)ceil_div((int64_t)3 << sh, 64), (unsigned)ceil_div(N, (int64_t)1 << sh));
+        hipLaunchKernelGGL(k_place_merge, mg, dim3(PT), 0, st, L.part, direct ? nullptr : L.chunk,
+                           place_direct(V), N, sh, L.H);
+        rc = check_launch("k_place_merge");
+    } else {
+        if (V > 0) {
+            hipLaunchKernelGGL(k_trace_keys, dim3((unsigned)ceil_div(V, TB)), dim3(TB), 0, st, bin,
+                               V, N, L.k0, L.v0);
+            rc = check_launch("k_trace_keys");
+            if (rc)
+                return rc;
+            size_t tb = L.cub_bytes;
+            if (hipcub::DeviceRadixSort::SortPairs(L.cub, tb, L.k0, L.k1, L.v0, L.v1, (int)V, 0,
+                                                   key_bits(N), st) != hipSuccess) {
+                set_error("lem_time_trace: radix sort failed");
+                return E_HIP;
+            }
+        }
+        hipLaunchKernelGGL(k_trace_starts, dim3((unsigned)ceil_div(N + 1, TB)), dim3(TB), 0, st,
+                           L.k1, V, N, L.start);
+        hipLaunchKernelGGL(k_trace_hist, dim3((unsigned)ceil_div(N, TB / 64)), dim3(TB), 0, st,
+                           amp, L.v1, L.start, N, L.H);
+        rc = check_launch("k_trace_hist");
     }
-    hipLaunchKernelGGL(k_trace_starts, dim3((unsigned)ceil_div(N + 1, TB)), dim3(TB), 0, st,
-                       L.k1, V, N, L.start);
-    LEM_REQUIRE(ceil_div(N, TB / 64) <= 2147483647LL, "lem_time_trace: too many samples");
-    hipLaunchKernelGGL(k_trace_hist, dim3((unsigned)ceil_div(N, TB / 64)), dim3(TB), 0, st, amp,
-                       L.v1, L.start, N, L.H);
-    hipLaunchKernelGGL(k_trace_conv, dim3((unsigned)ceil_div(N, TB)), dim3(TB), 0, st, L.H,
+    if (rc)
+        return rc;
+    hipLaunchKernelGGL(k_trace_conv, dim3((unsigned)ceil_div(N, 64)), dim3(PT), 0, st, L.H,
                        excitation, E, N, out);
     return check_launch("k_trace_conv");
 }
