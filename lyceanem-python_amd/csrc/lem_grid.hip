@@ -21,6 +21,7 @@
 // accepts always sits in a visited cell.
 #include "lem_device.h"
 #include "lem_field_dev.h"
+#include "lem_beam_walk.h"
 #include "lem_grid_walk.h"
 #include "lem_internal.h"
 #include "../../include/lem.h"
@@ -343,6 +344,9 @@ __global__ __launch_bounds__(GB) void k_visibility_grid(
 }
 
 constexpr int LDS_WG_PER_CU = 6;  // 6 x 25.5 KB of the 160 KB LDS of a CU
+// The beam walk: 96 registers, some spilled; at 4 (128 registers, none) the terrain
+// of beam_cast's figures takes 22.6 ms instead of 21.6.
+constexpr int BEAM_WPC = 5;
 // Any-hit walks whose macro table has at most MACRO_LDS_MAX7 blocks run 7
 // workgroups per CU (7 x 21.8 KB of LDS, 72 registers): the C3 one-bounce
 // masks gain 4 %.  The closest-hit walk keeps 6: at 72 registers it spills
@@ -434,13 +438,149 @@ constexpr int COUNTER_STRIDE = 512;  // uint64 elements
 // 1,083 / 1,089 / 1,093 ms and C3 (one bounce) 758 / 738 / 736 / 733 / 732 ms.
 constexpr int CLAIM_WORDS = 12;
 
+// Box of the points of each word of 64 lane slots: box[word] = lo, hi; counts the
+// narrow ones, whose two longest sides span at most BEAM_NARROW macro blocks together.
+// One wavefront a word.
+constexpr float BEAM_NARROW = 2.0f;
+__global__ __launch_bounds__(GB) void k_word_boxes(const float *__restrict__ p, int64_t n,
+                                                   const int32_t *__restrict__ order, GridDev G,
+                                                   float *__restrict__ box,
+                                                   unsigned long long *__restrict__ narrow)
+{
+    const int64_t slot = (int64_t)blockIdx.x * GB + threadIdx.x;
+    if ((slot & ~63ll) >= n)
+        return;  // wave-uniform
+    const int64_t at = slot < n ? slot : n - 1;  // lanes past the end repeat the last
+    const int64_t i = order ? (int64_t)order[at] : at;
+    float v[6] = {p[3 * i], p[3 * i + 1], p[3 * i + 2], -p[3 * i], -p[3 * i + 1], -p[3 * i + 2]};
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1)
+            v[c] = fminf(v[c], __shfl_xor(v[c], off));
+        if ((threadIdx.x & 63) == 0)
+            box[6 * (slot >> 6) + c] = c < 3 ? v[c] : -v[c];
+    }
+    const float inv = 1.0f / (float)(1 << G.mshift);
+    const float x = -(v[3] + v[0]) * G.icx * inv, y = -(v[4] + v[1]) * G.icy * inv,
+                z = -(v[5] + v[2]) * G.icz * inv;
+    const float area = fmaxf(x * y, fmaxf(x * z, y * z));
+    if ((threadIdx.x & 63) == 0 && area <= BEAM_NARROW)
+        atomicAdd(narrow, 1ull);
+}
+
+constexpr int BEAM_WORDS = 4;  // words whose beams a wavefront finds at once, 16 lanes each
+constexpr int BEAM_LIST = 16;  // blocks of a word's list
+
+// x of the lane `off` below in the row of 16, 0 at its start
+template <int OFF>
+LEM_DEV int row_below(int x)
+{
+    return __builtin_amdgcn_update_dpp(0, x, 0x110 + OFF, 0xf, 0xf, false);
+}
+
+// The beams of the words w0 .. w0 + 3 (below w1) to the point P: list[word][i] the macro
+// blocks to visit, in the rays' order, as (x | y << 16, z).  Returns, in the 16 lanes of
+// each word, how many there are; -1 if the rays walk one by one.  Sixteen slabs at a
+// time, a slab a lane: the arithmetic of one beam is the same in all its lanes, so four
+// words share its cost.
+LEM_DEV int beam_lists(const GridDev &G, const MacroTab &smq, const float *__restrict__ word_box,
+                       int64_t w0, int64_t w1, float px, float py, float pz, bool from_p,
+                       uint2 (*list)[BEAM_LIST])
+{
+    const int lane = threadIdx.x & 63, q = lane >> 4, l = lane & 15;
+    const int64_t w = w0 + q < w1 ? w0 + q : w1 - 1;
+    const float *wb = word_box + 6 * w;
+    const float x0 = wb[0], y0 = wb[1], z0 = wb[2], x1 = wb[3], y1 = wb[4], z1 = wb[5];
+    Beam b;
+    bool ok = beam_of(G, px, py, pz, x0, y0, z0, x1, y1, z1, from_p, b);
+    if (!ok)
+        b.slabs = 0;
+    int count = 0;
+    if (__ballot(b.slabs > 0)) {
+        const BeamAxis x = beam_axis(px, x0 - px, x1 - px, b.mrg),
+                       y = beam_axis(py, y0 - py, y1 - py, b.mrg),
+                       z = beam_axis(pz, z0 - pz, z1 - pz, b.mrg);
+        for (int base = 0; __ballot(base < b.slabs); base += 16) {
+            const int i = base + l, j = b.first + b.step * i;
+            int a0 = 0, na = 0, b0 = 0, nb = 0;
+            int n = i < b.slabs ? beam_slab(b, j, a0, na, b0, nb) : 0;
+            // one slab too wide: the whole word walks ray by ray
+            const bool wide = (n > BEAM_MAX) | (na > BEAM_NA) | (nb > BEAM_NB);
+            if (((__ballot(wide) >> (lane & 48)) & 0xffffull) != 0) {
+                ok = false;
+                b.slabs = n = 0;
+            }
+            uint32_t mask = beam_mask(G, smq, b.axis, x, y, z, j, a0, na, b0, n);
+            const int c = __popc(mask);
+            int s = c;
+            s += row_below<1>(s);
+            s += row_below<2>(s);
+            s += row_below<4>(s);
+            s += row_below<8>(s);
+            for (int at = count + s - c; mask != 0; mask &= mask - 1, ++at) {
+                const int bit = __builtin_ctz(mask);
+                int jx, jy, jz;
+                beam_block_at(b.axis, j, a0 + (bit & 7), b0 + (bit >> 3), jx, jy, jz);
+                if (at < BEAM_LIST)
+                    list[q][at] = make_uint2((uint32_t)jx | ((uint32_t)jy << 16), (uint32_t)jz);
+            }
+            count += __shfl(s, lane | 15);
+        }
+    }
+    return ok && count <= BEAM_LIST ? count : -1;
+}
+
+// The wavefront's rays through the n blocks of its word's list.
+//
+// A terrain of 10^6 triangles, 1,024 x 1,024 sources 30 m up, 512 sinks, closest hit:
+// 37.1 ms one by one, 3,320 vector instructions a word of 64 rays; 21.6 ms as beams,
+// 1,370 of them (290 for the lists).  What bounds it now is the gather of cell boxes
+// and triangles: the address units are busy 65 % of the time, with 56 loads a word
+// (77 one by one).  (Measured and left: the next cell's box loaded before this one's
+// triangles are tested, the same; one word's beam at a time over 64 lanes, 26.1 ms.)
+template <bool ANY, int SEM>
+LEM_DEV bool beam_cast(bool walk, const Ray &r, const Ray &rt, const GridDev &G,
+                       const int32_t *__restrict__ cell_start, const float4 *__restrict__ recs,
+                       const float4 *__restrict__ box, const MacroTab &smq, const uint2 *list, int n,
+                       float &dist)
+{
+    const RaySlabs k = ray_slabs(r);
+    RayHits h;
+    h.dist = r.len;
+    h.tmin = (double)r.len;
+    h.t_next = __builtin_huge_val();
+    h.id_min = -1;
+    h.hit = false;
+    for (int i = 0; i < n; ++i) {
+        const uint2 e = list[i];
+        const int xy = __builtin_amdgcn_readfirstlane((int)e.x),
+                  jz = __builtin_amdgcn_readfirstlane((int)e.y);
+        const int jx = xy & 0xffff, jy = (int)((uint32_t)xy >> 16);
+        if (walk)
+            block_walk<ANY, SEM>(r, rt, k, G, smq[(jz * G.my + jy) * G.mx + jx], jx, jy, jz, recs,
+                                 box, h);
+        if (ANY && !__ballot(walk && !h.hit))
+            break;
+    }
+    if (!ANY && SEM == 0 && h.hit) {
+        const float fs = (float)h.tmin;
+        const double delta = 8.0 * (2e-7 + (double)(nextafterf(fs, __builtin_huge_valf()) - fs));
+        if (h.t_next <= h.tmin + delta)
+            h.dist = replay_window(r, h.tmin, G, cell_start, recs);
+    }
+    dist = h.dist;
+    return h.hit;
+}
+
 // Persistent form of k_visibility_grid: each workgroup copies the quantised
 // macro table (at most lds_table(WPC) blocks) into LDS once; then each
 // wavefront repeatedly claims a 64-ray word of output (one atomic on one of
 // the 8 counters next_task[0..7]), so waves never wait for one another and
 // the load balances whatever number of workgroups is resident.  Dead-block
-// tests read LDS.  WPC: workgroups per CU the registers are bounded for.
-template <bool ANY, bool SINK_MAJOR, int SEM, bool REV = false, int WPC = LDS_WG_PER_CU>
+// tests read LDS.  WPC: workgroups per CU the registers are bounded for.  BEAM: the
+// words' rays walk as beams (lem_beam_walk.h) where their words allow it.
+template <bool ANY, bool SINK_MAJOR, int SEM, bool REV, int WPC, bool BEAM>
 __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
     const float *__restrict__ src, int64_t S, const float *__restrict__ snk, int64_t K, GridDev G,
     const int32_t *__restrict__ cell_start, const float4 *__restrict__ recs,
@@ -448,8 +588,17 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
     const int32_t *__restrict__ order, unsigned long long *__restrict__ bits,
     float *__restrict__ dist_out, unsigned long long *__restrict__ next_task, int skip_self,
     unsigned long long *__restrict__ par_count, uint2 *__restrict__ par_queue, int64_t par_cap,
-    int perm, const int32_t *__restrict__ outer_order)
+    int perm, const int32_t *__restrict__ outer_order, const float *__restrict__ word_box,
+    const unsigned long long *__restrict__ narrow)
 {
+    // both walks are launched where beams may serve; the words' boxes decide
+    if constexpr (!REV && SEM == LEM_SEM_NUMBA)
+        if (narrow) {
+            const int64_t words = ((SINK_MAJOR ? S : K) + 63) / 64;
+            if ((2 * (int64_t)*narrow >= words) != BEAM)
+                return;
+        }
+    __shared__ uint2 s_list[BEAM ? GB / 64 * BEAM_WORDS : 1][BEAM_LIST];
     __shared__ uint32_t smqa[lds_table(WPC)];
     __shared__ uint16_t smqb[lds_table(WPC)];
     __shared__ float4 saxis[3];
@@ -524,7 +673,8 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
         const int64_t w0 = owner * CH + u * CLAIM_WORDS;
         const int64_t end = (int64_t)(owner + 1) * CH < W ? (int64_t)(owner + 1) * CH : W;
         const int64_t w1 = w0 + CLAIM_WORDS < end ? w0 + CLAIM_WORDS : end;
-        for (int64_t word = w0; word < w1; ++word) {
+        // one word of 64 rays; n: blocks of its beam's list (-1: walk one by one)
+        auto cast_word = [&](int64_t word, int n, const uint2 *list) {
             const int64_t slot = word * 64 + lane;
             const bool active = slot < NI;
             // with an order, lane slot -> the slot-th point of the spatial order
@@ -535,29 +685,34 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
                            snk[3 * k + 1], snk[3 * k + 2]);
             float dist = r.len;
             bool hit = false;
-            if (active && !(skip_self && s == k)) {
-                // REV: walk from the sink end, test with the charged ray r
-                const Ray rw = REV ? charge(snk[3 * k], snk[3 * k + 1], snk[3 * k + 2],
-                                            src[3 * s], src[3 * s + 1], src[3 * s + 2])
-                                   : r;
+            // REV: walk from the sink end, test with the charged ray r
+            const Ray rw = REV ? charge(snk[3 * k], snk[3 * k + 1], snk[3 * k + 2], src[3 * s],
+                                        src[3 * s + 1], src[3 * s + 2])
+                               : r;
+            bool walk = active && !(skip_self && s == k) && n != 0;
+            // rays along a grid plane need the general slab test: they are
+            // queued for k_visibility_grid_par (left unblocked, at full
+            // length, here), which keeps that walk's registers and code out
+            // of this kernel
+            if (walk && (rw.dx == 0.0f || rw.dy == 0.0f || rw.dz == 0.0f)) {
+                walk = false;
+                // past the capacity the count only has to stay above it
+                if (__atomic_load_n(par_count, __ATOMIC_RELAXED) <= (unsigned long long)par_cap) {
+                    const unsigned long long q = atomicAdd(par_count, 1ull);
+                    if (q < (unsigned long long)par_cap)
+                        par_queue[q] = make_uint2((unsigned int)outer, (unsigned int)slot);
+                }
+            }
+            if (BEAM && n >= 0) {
+                // a source on its sink has no direction and meets nothing
+                if (n > 0)
+                    hit = beam_cast<ANY, SEM>(walk && rw.len > 0.0f, rw, r, G, cell_start, recs, box,
+                                              smq, list, n, dist);
+            } else if (walk) {
                 float dw = rw.len;
                 float &dd = REV ? dw : dist;
-                const Ray *rt = REV ? &r : nullptr;
-                // rays along a grid plane need the general slab test: they are
-                // queued for k_visibility_grid_par (left unblocked, at full
-                // length, here), which keeps that walk's registers and code out
-                // of this kernel
-                if (rw.dx == 0.0f || rw.dy == 0.0f || rw.dz == 0.0f) {
-                    // past the capacity the count only has to stay above it
-                    if (__atomic_load_n(par_count, __ATOMIC_RELAXED) <= (unsigned long long)par_cap) {
-                        const unsigned long long q = atomicAdd(par_count, 1ull);
-                        if (q < (unsigned long long)par_cap)
-                            par_queue[q] = make_uint2((unsigned int)outer, (unsigned int)slot);
-                    }
-                } else {
-                    hit = dda_cast<ANY, SEM, true, false>(rw, dd, G, cell_start, recs, box,
-                                                          nullptr, nullptr, nullptr, smq, rt);
-                }
+                hit = dda_cast<ANY, SEM, true, false>(rw, dd, G, cell_start, recs, box, nullptr,
+                                                      nullptr, nullptr, smq, REV ? &r : nullptr);
             }
             if (order && !perm) {
                 // the lanes' bits belong to several words (zeroed beforehand)
@@ -572,14 +727,30 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
             }
             if (dist_out && active)
                 dist_out[outer * NI + inner] = dist;
+        };
+        if constexpr (BEAM) {
+            const float *P = SINK_MAJOR ? snk + 3 * outer : src + 3 * outer;
+            uint2 (*list)[BEAM_LIST] = s_list + (threadIdx.x >> 6) * BEAM_WORDS;
+            for (int64_t word = w0; word < w1; word += BEAM_WORDS) {
+                const int cnt = beam_lists(G, smq, word_box, word, w1, P[0], P[1], P[2],
+                                           SINK_MAJOR == REV, list);
+                __builtin_amdgcn_wave_barrier();
+                const int64_t left = w1 - word;
+                for (int q = 0; q < BEAM_WORDS && q < left; ++q)
+                    cast_word(word + q, __builtin_amdgcn_readlane(cnt, 16 * q), list[q]);
+                __builtin_amdgcn_wave_barrier();
+            }
+        } else {
+            for (int64_t word = w0; word < w1; ++word)
+                cast_word(word, -1, nullptr);
         }
     }
 }
 
-// clears the 8 task counters of the persistent traversal
+// clears the 8 task counters of the persistent traversal and the count of narrow words
 __global__ void k_zero_u64(unsigned long long *__restrict__ p)
 {
-    if (threadIdx.x < 8)
+    if (threadIdx.x < 9)
         p[threadIdx.x * COUNTER_STRIDE] = 0ull;
 }
 
@@ -749,7 +920,8 @@ struct VisWs {
 };
 
 constexpr int MORTON_BITS = 30;
-// workspace head: the 8 task counters (4 KB apart), then the point bounds
+// workspace head: the 8 task counters (4 KB apart), then the point bounds (afterwards
+// the count of narrow words)
 constexpr int64_t VIS_HEAD = 8 * 8 * COUNTER_STRIDE + 256;
 
 inline int64_t vis_sort_bytes(int64_t n)
@@ -1252,6 +1424,25 @@ extern "C" int lem_visibility_grid(const float *src, int64_t S, const float *snk
         const int64_t nwg =
             std::max<int64_t>(1, std::min<int64_t>(ceil_div(words, 4), (int64_t)cus * per_cu));
         hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, L.counter);
+        // Beams serve rays in a spatial order whose words are narrow (k_word_boxes) and
+        // that go on past the first blocks: not those walked from the sink end, whose
+        // hits are near it (5,000 to 50,000 triangles, 3,600 sources x 30,000 sinks:
+        // 3.37 and 5.74 ms one by one, 3.43 and 6.03 as beams).  BEAM_NARROW: the same
+        // triangles, 30,000 sources to a plate of 33 x 33 sinks, 2.5 and 11 square
+        // blocks a word, 2.56 and 7.45 ms one by one, 2.91 and 8.65 as beams; terrain of
+        // 10^6 triangles, 512 sinks, words of 0.08, 0.3, 1.3 and 5 square blocks: 37.1,
+        // 14.4, 7.4 and 6.0 -> 21.7, 9.8, 5.5 and 4.9.  Below 2^22 rays the boxes and
+        // the launch are not worth it.  The boxes take the place of the Morton keys.
+        float *word_box = nullptr;
+        unsigned long long *narrow = nullptr;
+        if (order && !rev && semantics != LEM_SEM_NATIVE && (double)S * (double)K >= 4194304.0) {
+            word_box = reinterpret_cast<float *>(L.k0);
+            narrow = L.counter + 8 * COUNTER_STRIDE;
+            hipLaunchKernelGGL(k_word_boxes, dim3((unsigned)nbl), dim3(GB), 0, st,
+                               sink_major ? src : snk, NI, order, G, word_box, narrow);
+        }
+        const int64_t nbeam =
+            std::max<int64_t>(1, std::min<int64_t>(ceil_div(words, 4), (int64_t)cus * BEAM_WPC));
         // queue of the rays along grid planes, walked afterwards by
         // k_visibility_grid_par over as many workgroups as fill the chip
         char *qb = reinterpret_cast<char *>(workspace) + (need - PAR_QUEUE_BYTES);
@@ -1260,10 +1451,18 @@ extern "C" int lem_visibility_grid(const float *src, int64_t S, const float *snk
         hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(GB), 0, st, pcount, 1);
 #define LEM_VGL(A, M, SM, R, WP)                                                              \
     do {                                                                                      \
-        hipLaunchKernelGGL((k_visibility_grid_lds<A, M, SM, R, WP>), dim3((unsigned)nwg), dim3(GB), 0, \
-                           st, src, S, snk, K, G, cell_start, rc4, bx4, mq, info->nmacro, order, \
-                           hb, dist, L.counter, skip_self, pcount, pq, PAR_QUEUE_CAP,          \
-                           perm ? 1 : 0, outer_order);                                         \
+        if constexpr (!R && SM == LEM_SEM_NUMBA) {                                            \
+            if (word_box)                                                                     \
+                hipLaunchKernelGGL((k_visibility_grid_lds<A, M, SM, R, BEAM_WPC, true>),      \
+                                   dim3((unsigned)nbeam), dim3(GB), 0, st, src, S, snk, K, G, \
+                                   cell_start, rc4, bx4, mq, info->nmacro, order, hb, dist,   \
+                                   L.counter, skip_self, pcount, pq, PAR_QUEUE_CAP, perm ? 1 : 0, \
+                                   outer_order, word_box, narrow);                            \
+        }                                                                                     \
+        hipLaunchKernelGGL((k_visibility_grid_lds<A, M, SM, R, WP, false>), dim3((unsigned)nwg), \
+                           dim3(GB), 0, st, src, S, snk, K, G, cell_start, rc4, bx4, mq,      \
+                           info->nmacro, order, hb, dist, L.counter, skip_self, pcount, pq,   \
+                           PAR_QUEUE_CAP, perm ? 1 : 0, outer_order, nullptr, narrow);        \
         hipLaunchKernelGGL((k_visibility_grid_par<A, M, SM, R>), dim3((unsigned)nwg), dim3(GB), 0, \
                            st, src, S, snk, K, G, cell_start, rc4, bx4, mq, info->nmacro, order, \
                            hb, dist, skip_self, pcount, pq, PAR_QUEUE_CAP, perm ? 1 : 0);      \
