@@ -60,8 +60,11 @@ __global__ void k_bounds_init(unsigned int *b)
         b[threadIdx.x] = 0u;  // max keys
 }
 
-__global__ __launch_bounds__(GB) void k_bounds(const float *__restrict__ tris, int64_t n_vals,
-                                               unsigned int *__restrict__ b)
+// Bound by its atomics, one behind the other on each of the six words: few large
+// workgroups (3 M vertices: 4,096 of 256 threads 98 us, 256 of 1,024 13).
+constexpr int BOUNDS_TB = 1024, BOUNDS_BLOCKS = 256;
+__global__ __launch_bounds__(BOUNDS_TB) void k_bounds(const float *__restrict__ tris,
+                                                      int64_t n_vals, unsigned int *__restrict__ b)
 {
     __shared__ unsigned int smin[3], smax[3];
     if (threadIdx.x < 3) {
@@ -72,14 +75,22 @@ __global__ __launch_bounds__(GB) void k_bounds(const float *__restrict__ tris, i
     unsigned int lmin[3] = {0xffffffffu, 0xffffffffu, 0xffffffffu};
     unsigned int lmax[3] = {0u, 0u, 0u};
     // n_vals = 3 * number of vertices; value i has axis i % 3
-    for (int64_t v = (int64_t)blockIdx.x * GB + threadIdx.x; v * 3 < n_vals;
-         v += (int64_t)gridDim.x * GB) {
+    const int64_t nv = n_vals / 3, stride = (int64_t)gridDim.x * BOUNDS_TB;
+    for (int64_t v = (int64_t)blockIdx.x * BOUNDS_TB + threadIdx.x; v < nv; v += 4 * stride) {
+        float x[4][3];  // four vertices in flight; past the end the first again
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            unsigned int k = fkey(tris[3 * v + a]);
-            lmin[a] = k < lmin[a] ? k : lmin[a];
-            lmax[a] = k > lmax[a] ? k : lmax[a];
-        }
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+                x[q][a] = tris[3 * (v + q * stride < nv ? v + q * stride : v) + a];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                const unsigned int k = fkey(x[q][a]);
+                lmin[a] = k < lmin[a] ? k : lmin[a];
+                lmax[a] = k > lmax[a] ? k : lmax[a];
+            }
     }
     // wave minima / maxima first, then one LDS atomic per wave and bound
 #pragma unroll
@@ -104,18 +115,75 @@ __global__ __launch_bounds__(GB) void k_bounds(const float *__restrict__ tris, i
     }
 }
 
+inline unsigned bounds_blocks(int64_t nv)
+{
+    return (unsigned)std::min<int64_t>(ceil_div(nv, BOUNDS_TB), BOUNDS_BLOCKS);
+}
+
+// Cells of a triangle one by one (cell -1: none left), in step over the wavefront.
+struct CellWalk {
+    int lo[3], hi[3], x, y, z;
+};
+
+LEM_DEV CellWalk cell_walk(const float *__restrict__ tris, int64_t t, int64_t T, const GridDev &G)
+{
+    CellWalk w;
+    w.lo[0] = w.lo[1] = w.lo[2] = 0;
+    w.hi[0] = w.hi[1] = w.hi[2] = -1;
+    if (t < T)
+        tri_cell_range(G, tris + 9 * t, w.lo, w.hi);
+    w.x = w.lo[0];
+    w.y = w.lo[1];
+    w.z = w.lo[2];
+    return w;
+}
+
+LEM_DEV int next_cell(CellWalk &w, const GridDev &G)
+{
+    if (w.z > w.hi[2])
+        return -1;
+    const int c = (w.z * G.ny + w.y) * G.nx + w.x;  // at most 10^9 cells
+    if (++w.x > w.hi[0]) {
+        w.x = w.lo[0];
+        if (++w.y > w.hi[1]) {
+            w.y = w.lo[1];
+            ++w.z;
+        }
+    }
+    return c;
+}
+
+// counters[cell] += 1 for every lane with a cell, one atomic for each run of lanes with
+// the same one (neighbouring triangles of a mesh share cells, and atomics on one word
+// come one behind the other); returns the lane's own earlier value (SLOT).
+template <bool SLOT>
+LEM_DEV int count_cells(int *__restrict__ counters, int cell)
+{
+    const int lane = threadIdx.x & 63;
+    const int before = __shfl_up(cell, 1);
+    const bool head = lane == 0 || cell != before;
+    const unsigned long long heads = __ballot(head);
+    const unsigned long long upto = (2ull << lane) - 1;  // lanes 0 .. lane (lane 63: all)
+    int slot = 0;
+    if (head && cell >= 0) {
+        const unsigned long long later = heads & ~upto;
+        slot = atomicAdd(&counters[cell], (later ? (int)__builtin_ctzll(later) : 64) - lane);
+    }
+    if (SLOT) {
+        const int first = 63 - (int)__builtin_clzll(heads & upto);
+        slot = __shfl(slot, first) + lane - first;
+    }
+    return slot;
+}
+
+// Bound by the atomics: 10^6 triangles of a terrain, 2.28 M references, 15 us (one
+// atomic each: 92).
 __global__ __launch_bounds__(GB) void k_count(const float *__restrict__ tris, int64_t T, GridDev G,
                                               int *__restrict__ counts)
 {
-    int64_t t = (int64_t)blockIdx.x * GB + threadIdx.x;
-    if (t >= T)
-        return;
-    int lo[3], hi[3];
-    tri_cell_range(G, tris + 9 * t, lo, hi);
-    for (int z = lo[2]; z <= hi[2]; ++z)
-        for (int y = lo[1]; y <= hi[1]; ++y)
-            for (int x = lo[0]; x <= hi[0]; ++x)
-                atomicAdd(&counts[((int64_t)z * G.ny + y) * G.nx + x], 1);
+    CellWalk w = cell_walk(tris, (int64_t)blockIdx.x * GB + threadIdx.x, T, G);
+    for (int c = next_cell(w, G); __ballot(c >= 0); c = next_cell(w, G))
+        count_cells<false>(counts, c);
 }
 
 // Exclusive scan, three phases: per-block scan + block sums, scan of the block
@@ -191,23 +259,49 @@ __global__ __launch_bounds__(GB) void k_starts(const long long *__restrict__ sca
     }
 }
 
+// As k_count (one atomic each: 110 us, this 19).
 __global__ __launch_bounds__(GB) void k_fill(const float *__restrict__ tris, int64_t T, GridDev G,
                                              int *__restrict__ cursor, int32_t *__restrict__ ids)
 {
-    int64_t t = (int64_t)blockIdx.x * GB + threadIdx.x;
-    if (t >= T)
-        return;
-    int lo[3], hi[3];
-    tri_cell_range(G, tris + 9 * t, lo, hi);
-    for (int z = lo[2]; z <= hi[2]; ++z)
-        for (int y = lo[1]; y <= hi[1]; ++y)
-            for (int x = lo[0]; x <= hi[0]; ++x) {
-                int slot = atomicAdd(&cursor[((int64_t)z * G.ny + y) * G.nx + x], 1);
-                ids[slot] = (int32_t)t;
-            }
+    const int64_t t = (int64_t)blockIdx.x * GB + threadIdx.x;
+    CellWalk w = cell_walk(tris, t, T, G);
+    for (int c = next_cell(w, G); __ballot(c >= 0); c = next_cell(w, G)) {
+        const int slot = count_cells<true>(cursor, c);
+        if (c >= 0)
+            ids[slot] = (int32_t)t;
+    }
 }
 
-// Each cell's ids in increasing triangle order (shell sort; lists are short).
+// n <= N ids in increasing order: Batcher's odd-even merge sort in registers, every
+// load in flight at once.
+template <int N>
+LEM_DEV void sort_ids(int32_t *a, int n)
+{
+    int32_t v[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+        v[i] = i < n ? a[i] : 0x7fffffff;
+#pragma unroll
+    for (int p = 1; p < N; p *= 2)
+#pragma unroll
+        for (int k = p; k >= 1; k /= 2)
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+                if (i + k < N && i >= k % p && (i - k % p) % (2 * k) < k &&
+                    i / (2 * p) == (i + k) / (2 * p)) {
+                    const int32_t lo = min(v[i], v[i + k]), hi = max(v[i], v[i + k]);
+                    v[i] = lo;
+                    v[i + k] = hi;
+                }
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+        if (i < n)
+            a[i] = v[i];
+}
+
+// Each cell's ids in increasing triangle order: up to 32 in registers (10^6 triangles
+// of a terrain, 130,000 cells of mostly 18 to 32: 16 us; a shell sort in memory, a
+// dependent load a step: 114), more by the shell sort.
 __global__ __launch_bounds__(GB) void k_sort_cells(const int32_t *__restrict__ cell_start,
                                                    int64_t ncells, int32_t *__restrict__ ids)
 {
@@ -216,6 +310,16 @@ __global__ __launch_bounds__(GB) void k_sort_cells(const int32_t *__restrict__ c
         return;
     int32_t b = cell_start[c], n = cell_start[c + 1] - b;
     int32_t *a = ids + b;
+    if (n < 2)
+        return;
+    if (n <= 8) {
+        sort_ids<8>(a, n);
+        return;
+    }
+    if (n <= 32) {
+        sort_ids<32>(a, n);
+        return;
+    }
     for (int gap = n / 2; gap > 0; gap /= 2) {
         for (int i = gap; i < n; ++i) {
             int32_t v = a[i];
@@ -255,28 +359,34 @@ __global__ __launch_bounds__(GB) void k_cell_boxes(const float *__restrict__ tri
     cell_box_of(tris, cell_start, ids, G, c, box[2 * c], box[2 * c + 1]);
 }
 
-// Macro-block boxes, written after the ncells cell boxes.
-__global__ __launch_bounds__(GB) void k_macro_boxes(GridDev G, float4 *__restrict__ box)
-{
-    const int64_t m = (int64_t)blockIdx.x * GB + threadIdx.x;
-    const int64_t nm = (int64_t)G.mx * G.my * G.mz;
-    if (m >= nm)
-        return;
-    float4 lo, hi;
-    macro_box_of(G, box, m, lo, hi);
-    box[2 * (G.ncells + m)] = lo;
-    box[2 * (G.ncells + m) + 1] = hi;
-}
-
-// Quantised macro table (8 bytes a block).
-__global__ __launch_bounds__(GB) void k_macro_quant(GridDev G, const float4 *__restrict__ box,
+// Macro-block boxes, written after the ncells cell boxes, and their quantised form (8
+// bytes a block).  A wavefront a block: it reads up to 2^(3 mshift) cell boxes, of
+// which one lane keeps too few in flight (3,844 blocks of 512 cells: 245 us, this
+// 13).
+__global__ __launch_bounds__(GB) void k_macro_boxes(GridDev G, float4 *__restrict__ box,
                                                     uint2 *__restrict__ mq)
 {
-    const int64_t m = (int64_t)blockIdx.x * GB + threadIdx.x;
+    const int64_t m = (int64_t)blockIdx.x * (GB / 64) + (threadIdx.x >> 6);
     const int64_t nm = (int64_t)G.mx * G.my * G.mz;
     if (m >= nm)
-        return;
-    mq[m] = macro_quant_of(G, box, m);
+        return;  // wave-uniform
+    const int lane = threadIdx.x & 63;
+    float4 lo, hi;
+    macro_box_of(G, box, m, lane, 64, lo, hi);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        lo.x = fminf(lo.x, __shfl_xor(lo.x, off));
+        lo.y = fminf(lo.y, __shfl_xor(lo.y, off));
+        lo.z = fminf(lo.z, __shfl_xor(lo.z, off));
+        hi.x = fmaxf(hi.x, __shfl_xor(hi.x, off));
+        hi.y = fmaxf(hi.y, __shfl_xor(hi.y, off));
+        hi.z = fmaxf(hi.z, __shfl_xor(hi.z, off));
+    }
+    if (lane == 0) {
+        box[2 * (G.ncells + m)] = lo;
+        box[2 * (G.ncells + m) + 1] = hi;
+        mq[m] = macro_quant_of(G, lo, hi, m);
+    }
 }
 
 // Dense S x K through the grid.
@@ -964,8 +1074,8 @@ int morton_order(const float *pts, int64_t n, const VisWs &L, hipStream_t st)
         hipLaunchKernelGGL(k_morton_small, dim3(1), dim3(MB), 0, st, pts, n, L.k0, L.v0);
     } else {
         hipLaunchKernelGGL(k_bounds_init, dim3(1), dim3(64), 0, st, L.bounds);
-        hipLaunchKernelGGL(k_bounds, dim3((unsigned)std::min<int64_t>(ceil_div(n, GB), 1024)),
-                           dim3(GB), 0, st, pts, 3 * n, L.bounds);
+        hipLaunchKernelGGL(k_bounds, dim3(bounds_blocks(n)), dim3(BOUNDS_TB), 0, st, pts, 3 * n,
+                           L.bounds);
         hipLaunchKernelGGL(k_morton_keys, dim3((unsigned)ceil_div(n, GB)), dim3(GB), 0, st, pts,
                            n, L.bounds, L.k0, L.v0);
     }
@@ -1188,8 +1298,8 @@ extern "C" int lem_grid_plan(const float *tris, int64_t T, float cells_per_tri,
     PlanWs L = plan_layout(workspace, cap);
     hipLaunchKernelGGL(k_bounds_init, dim3(1), dim3(64), 0, st, L.bounds);
     int64_t nvals = 9 * T;
-    int64_t nblk = std::min<int64_t>(ceil_div(3 * T, GB), 4096);
-    hipLaunchKernelGGL(k_bounds, dim3((unsigned)nblk), dim3(GB), 0, st, tris, nvals, L.bounds);
+    hipLaunchKernelGGL(k_bounds, dim3(bounds_blocks(3 * T)), dim3(BOUNDS_TB), 0, st, tris, nvals,
+                       L.bounds);
     int rc = check_launch("k_bounds");
     if (rc)
         return rc;
@@ -1266,10 +1376,8 @@ extern "C" int lem_grid_fill(const float *tris, int64_t T, const lem_grid_info *
                            tris, tri_ids, info->nrefs, reinterpret_cast<float4 *>(recs));
     hipLaunchKernelGGL(k_cell_boxes, dim3((unsigned)ceil_div(nc, GB)), dim3(GB), 0, st, tris,
                        cell_start, tri_ids, G, nc, reinterpret_cast<float4 *>(cell_box));
-    hipLaunchKernelGGL(k_macro_boxes, dim3((unsigned)ceil_div(info->nmacro, GB)), dim3(GB), 0, st,
-                       G, reinterpret_cast<float4 *>(cell_box));
-    hipLaunchKernelGGL(k_macro_quant, dim3((unsigned)ceil_div(info->nmacro, GB)), dim3(GB), 0, st,
-                       G, reinterpret_cast<const float4 *>(cell_box),
+    hipLaunchKernelGGL(k_macro_boxes, dim3((unsigned)ceil_div(info->nmacro, GB / 64)), dim3(GB), 0,
+                       st, G, reinterpret_cast<float4 *>(cell_box),
                        reinterpret_cast<uint2 *>(cell_box + 8 * (nc + info->nmacro)));
     return check_launch("lem_grid_fill");
 }

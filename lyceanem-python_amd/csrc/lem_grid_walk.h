@@ -664,7 +664,9 @@ LEM_DEV void cell_box_of(const float *__restrict__ tris, const int32_t *__restri
 {
     const float INF = __builtin_huge_valf();
     float lo[3] = {INF, INF, INF}, hi[3] = {-INF, -INF, -INF};
-    for (int32_t j = cell_start[c]; j < cell_start[c + 1]; ++j) {
+    const int32_t j1 = cell_start[c + 1];
+#pragma unroll 4
+    for (int32_t j = cell_start[c]; j < j1; ++j) {
         const float *t = tris + 9 * (int64_t)ids[j];
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
@@ -688,26 +690,36 @@ LEM_DEV void cell_box_of(const float *__restrict__ tris, const int32_t *__restri
     out_hi = make_float4(hi[0], hi[1], hi[2], __builtin_bit_cast(float, cell_start[c + 1]));
 }
 
-// Box of macro block m: the union of its cells' boxes (inverted if empty).
-LEM_DEV void macro_box_of(const GridDev &G, const float4 *__restrict__ box, int64_t m,
-                          float4 &out_lo, float4 &out_hi)
+// Box of macro block m: the union of its cells' boxes (inverted if empty).  Of its
+// cells only first, first + step, ...: a wavefront's lanes share a block.
+LEM_DEV void macro_box_of(const GridDev &G, const float4 *__restrict__ box, int64_t m, int first,
+                          int step, float4 &out_lo, float4 &out_hi)
 {
     const int jx = (int)(m % G.mx), jy = (int)((m / G.mx) % G.my), jz = (int)(m / ((int64_t)G.mx * G.my));
     const int B = 1 << G.mshift;
     const float INF = __builtin_huge_valf();
     float4 lo = make_float4(INF, INF, INF, 0.0f), hi = make_float4(-INF, -INF, -INF, 0.0f);
-    for (int z = jz * B; z < min((jz + 1) * B, G.nz); ++z)
-        for (int y = jy * B; y < min((jy + 1) * B, G.ny); ++y)
-            for (int x = jx * B; x < min((jx + 1) * B, G.nx); ++x) {
-                const int64_t c = ((int64_t)z * G.ny + y) * G.nx + x;
-                const float4 a = box[2 * c], b = box[2 * c + 1];
-                if (a.x <= b.x) {
-                    lo.x = fminf(lo.x, a.x); lo.y = fminf(lo.y, a.y); lo.z = fminf(lo.z, a.z);
-                    hi.x = fmaxf(hi.x, b.x); hi.y = fmaxf(hi.y, b.y); hi.z = fmaxf(hi.z, b.z);
-                }
-            }
+    for (int i = first; i < 1 << (3 * G.mshift); i += step) {
+        const int x = jx * B + (i & (B - 1)), y = jy * B + ((i >> G.mshift) & (B - 1)),
+                  z = jz * B + (i >> (2 * G.mshift));
+        if (x >= G.nx || y >= G.ny || z >= G.nz)
+            continue;
+        const int64_t c = ((int64_t)z * G.ny + y) * G.nx + x;
+        const float4 a = box[2 * c], b = box[2 * c + 1];
+        if (a.x <= b.x) {
+            lo.x = fminf(lo.x, a.x); lo.y = fminf(lo.y, a.y); lo.z = fminf(lo.z, a.z);
+            hi.x = fmaxf(hi.x, b.x); hi.y = fmaxf(hi.y, b.y); hi.z = fmaxf(hi.z, b.z);
+        }
+    }
     out_lo = lo;
     out_hi = hi;
+}
+
+// The whole of it.
+LEM_DEV void macro_box_of(const GridDev &G, const float4 *__restrict__ box, int64_t m,
+                          float4 &out_lo, float4 &out_hi)
+{
+    macro_box_of(G, box, m, 0, 1, out_lo, out_hi);
 }
 
 // Macro box m quantised to 8 bytes: per axis, lo and hi as steps of
@@ -718,10 +730,9 @@ LEM_DEV void macro_box_of(const GridDev &G, const float4 *__restrict__ box, int6
 // covers the part of the union box within eps of the block -- every hit point
 // the walk tests while it is in the block, also one on a block face that the
 // walk's rounding assigns to this block.
-LEM_DEV uint2 macro_quant_of(const GridDev &G, const float4 *__restrict__ box, int64_t m)
+LEM_DEV uint2 macro_quant_of(const GridDev &G, const float4 &lo, const float4 &hi, int64_t m)
 {
     const int jx = (int)(m % G.mx), jy = (int)((m / G.mx) % G.my), jz = (int)(m / ((int64_t)G.mx * G.my));
-    const float4 lo = box[2 * (G.ncells + m)], hi = box[2 * (G.ncells + m) + 1];
     if (!(lo.x <= hi.x))
         return make_uint2(0x00ffffffu, 0u);  // lo = 255 > hi = 0 on every axis
     const float o[3] = {macro_origin(G.qlx, G.cx, jx, G.mshift),
@@ -738,6 +749,11 @@ LEM_DEV uint2 macro_quant_of(const GridDev &G, const float4 *__restrict__ box, i
         qh[a] = (unsigned int)(fh < 0.0 ? 0.0 : (fh > 255.0 ? 255.0 : fh));
     }
     return make_uint2(ql[0] | (ql[1] << 8) | (ql[2] << 16) | (qh[0] << 24), qh[1] | (qh[2] << 8));
+}
+
+LEM_DEV uint2 macro_quant_of(const GridDev &G, const float4 *__restrict__ box, int64_t m)
+{
+    return macro_quant_of(G, box[2 * (G.ncells + m)], box[2 * (G.ncells + m) + 1], m);
 }
 
 // Cell budget of the plan (the count array's capacity).
