@@ -65,6 +65,18 @@ struct Beam {
     int first, step, slabs;    // slabs in the rays' direction
 };
 
+// What covers the rounding of every test of a beam: each is a handful of float32
+// operations on values up to the points' and their differences.
+LEM_DEV float beam_margin(const GridDev &G, float px, float py, float pz, float lox, float loy,
+                          float loz, float hix, float hiy, float hiz)
+{
+    const float far = fmaxf(fmaxf(fmaxf(fabsf(lox - px), fabsf(hix - px)),
+                                  fmaxf(fabsf(loy - py), fabsf(hiy - py))),
+                            fmaxf(fabsf(loz - pz), fabsf(hiz - pz)));
+    const float at = fmaxf(fmaxf(fabsf(px), fabsf(py)), fabsf(pz));
+    return 2.0f * G.eps + 1e-6f * (far + at);
+}
+
 // The beam from P to the box [lo, hi]; from_p: the rays start at P.  False: too
 // wide for it, or not finite (the rays then walk one by one).
 LEM_DEV bool beam_of(const GridDev &G, float px, float py, float pz, float lox, float loy, float loz,
@@ -75,11 +87,7 @@ LEM_DEV bool beam_of(const GridDev &G, float px, float py, float pz, float lox, 
     const int gmx = G.mx, gmy = G.my, gmz = G.mz;
     const float ax = lox - px, ay = loy - py, az = loz - pz;
     const float bx = hix - px, by = hiy - py, bz = hiz - pz;
-    const float far = fmaxf(fmaxf(fmaxf(fabsf(ax), fabsf(bx)), fmaxf(fabsf(ay), fabsf(by))),
-                            fmaxf(fabsf(az), fabsf(bz)));
-    const float at = fmaxf(fmaxf(fabsf(px), fabsf(py)), fabsf(pz));
-    // every test is a handful of float32 operations on values up to far + at
-    const float mrg = 2.0f * G.eps + 1e-6f * (far + at);
+    const float mrg = beam_margin(G, px, py, pz, lox, loy, loz, hix, hiy, hiz);
     if (!(mrg < 1e30f))
         return false;
     // blocks per unit (cells per unit times a power of two) and the ends in blocks
@@ -183,6 +191,50 @@ LEM_DEV uint32_t beam_mask(const GridDev &G, const MacroTab &smq, int axis, cons
         }
     }
     return mask;
+}
+
+// A pencil: a beam so narrow that its rays cross the same cells.  Then the cells are
+// found for all rays at once too, and every ray is tested with every triangle of them.
+// Sub-blocks of 4 x 4 x 4 cells, one cell a lane.
+
+// Sub-block s of block (jx, jy, jz): its first cell, and whether the beam meets it.
+LEM_DEV bool pencil_sub(const GridDev &G, const BeamAxis &x, const BeamAxis &y, const BeamAxis &z,
+                        int jx, int jy, int jz, int s, int &cx, int &cy, int &cz)
+{
+    const int b = G.mshift - 2, m = (1 << b) - 1;
+    cx = (jx << G.mshift) + ((s & m) << 2);
+    cy = (jy << G.mshift) + (((s >> b) & m) << 2);
+    cz = (jz << G.mshift) + ((s >> (2 * b)) << 2);
+    float u0 = 0.0f, u1 = 1.0f;
+    const float lx = __builtin_fmaf(G.cx, (float)cx, G.lox), ly = __builtin_fmaf(G.cy, (float)cy, G.loy),
+                lz = __builtin_fmaf(G.cz, (float)cz, G.loz);
+    beam_clip(x, lx, __builtin_fmaf(G.cx, 4.0f, lx), u0, u1);
+    beam_clip(y, ly, __builtin_fmaf(G.cy, 4.0f, ly), u0, u1);
+    beam_clip(z, lz, __builtin_fmaf(G.cz, 4.0f, lz), u0, u1);
+    return (u0 <= u1) & (cx < G.nx) & (cy < G.ny) & (cz < G.nz);
+}
+
+// Cell `l` of the sub-block whose first cell is (cx, cy, cz): its triangles [b, e), none
+// if the beam misses its box.  up_*: the rays' direction (cells come in their order).
+LEM_DEV void pencil_cell(const GridDev &G, const float4 *__restrict__ box, const BeamAxis &x,
+                         const BeamAxis &y, const BeamAxis &z, int cx, int cy, int cz, int l,
+                         bool up_x, bool up_y, bool up_z, int32_t &b, int32_t &e)
+{
+    const int ix = cx + ((l & 3) ^ (up_x ? 0 : 3)), iy = cy + (((l >> 2) & 3) ^ (up_y ? 0 : 3)),
+              iz = cz + ((l >> 4) ^ (up_z ? 0 : 3));
+    b = e = 0;
+    if ((ix >= G.nx) | (iy >= G.ny) | (iz >= G.nz))
+        return;
+    const int c = (iz * G.ny + iy) * G.nx + ix;
+    const float4 lo = box[2 * c], hi = box[2 * c + 1];
+    float u0 = 0.0f, u1 = 1.0f;
+    beam_clip(x, lo.x, hi.x, u0, u1);
+    beam_clip(y, lo.y, hi.y, u0, u1);
+    beam_clip(z, lo.z, hi.z, u0, u1);
+    if (u0 <= u1) {
+        b = __builtin_bit_cast(int32_t, lo.w);
+        e = __builtin_bit_cast(int32_t, hi.w);
+    }
 }
 
 // A ray's reciprocal direction and origin times it: the plane at x is t = x id + oid.

@@ -457,6 +457,7 @@ constexpr int LDS_WG_PER_CU = 6;  // 6 x 25.5 KB of the 160 KB LDS of a CU
 // The beam walk: 96 registers, some spilled; at 4 (128 registers, none) the terrain
 // of beam_cast's figures takes 22.6 ms instead of 21.6.
 constexpr int BEAM_WPC = 5;
+enum { WALK_RAY, WALK_BEAM, WALK_PENCIL };
 // Any-hit walks whose macro table has at most MACRO_LDS_MAX7 blocks run 7
 // workgroups per CU (7 x 21.8 KB of LDS, 72 registers): the C3 one-bounce
 // masks gain 4 %.  The closest-hit walk keeps 6: at 72 registers it spills
@@ -549,9 +550,10 @@ constexpr int COUNTER_STRIDE = 512;  // uint64 elements
 constexpr int CLAIM_WORDS = 12;
 
 // Box of the points of each word of 64 lane slots: box[word] = lo, hi; counts the
-// narrow ones, whose two longest sides span at most BEAM_NARROW macro blocks together.
-// One wavefront a word.
-constexpr float BEAM_NARROW = 2.0f;
+// narrow ones, whose two longest sides span at most BEAM_NARROW square macro blocks
+// (narrow[0]), and the pencils, at most BEAM_PENCIL square cells (narrow[1]).  One
+// wavefront a word.
+constexpr float BEAM_NARROW = 2.0f, BEAM_PENCIL = 0.25f;
 __global__ __launch_bounds__(GB) void k_word_boxes(const float *__restrict__ p, int64_t n,
                                                    const int32_t *__restrict__ order, GridDev G,
                                                    float *__restrict__ box,
@@ -575,8 +577,22 @@ __global__ __launch_bounds__(GB) void k_word_boxes(const float *__restrict__ p, 
     const float x = -(v[3] + v[0]) * G.icx * inv, y = -(v[4] + v[1]) * G.icy * inv,
                 z = -(v[5] + v[2]) * G.icz * inv;
     const float area = fmaxf(x * y, fmaxf(x * z, y * z));
-    if ((threadIdx.x & 63) == 0 && area <= BEAM_NARROW)
+    if ((threadIdx.x & 63) == 0 && area <= BEAM_NARROW) {
         atomicAdd(narrow, 1ull);
+        // pencil_sub's sub-blocks are at most 64
+        if (area <= BEAM_PENCIL * inv * inv && G.mshift >= 2 && G.mshift <= 4)
+            atomicAdd(narrow + 1, 1ull);
+    }
+}
+
+// The walk of a call, from its words: chosen = WALK_*.
+__global__ void k_choose_walk(const unsigned long long *__restrict__ narrow, int64_t words, int any,
+                              int rev, unsigned long long *__restrict__ chosen)
+{
+    if (threadIdx.x == 0)
+        *chosen = any && 2 * (int64_t)narrow[1] >= words    ? WALK_PENCIL
+                  : !rev && 2 * (int64_t)narrow[0] >= words ? WALK_BEAM
+                                                            : WALK_RAY;
 }
 
 constexpr int BEAM_WORDS = 4;  // words whose beams a wavefront finds at once, 16 lanes each
@@ -683,14 +699,61 @@ LEM_DEV bool beam_cast(bool walk, const Ray &r, const Ray &rt, const GridDev &G,
     return h.hit;
 }
 
+// As beam_cast for a pencil, any hit: the word's cells and their triangles are the same
+// for all its rays, so triangles come through scalar loads and every lane tests each.
+// 50,000 triangles, 3,600 sources x 30,001 sinks from the sink end: 5.74 ms one by one,
+// 2,615 vector instructions and 81 vector loads a word; 4.70 ms, 1,663 and 29.
+LEM_DEV bool pencil_cast(bool walk, const Ray &rt, const GridDev &G, const float4 *__restrict__ recs,
+                         const float4 *__restrict__ box, const float *__restrict__ wb, float px,
+                         float py, float pz, bool from_p, const uint2 *list, int n)
+{
+    const int lane = threadIdx.x & 63;
+    const float x0 = wb[0], y0 = wb[1], z0 = wb[2], x1 = wb[3], y1 = wb[4], z1 = wb[5];
+    const bool up_x = (x0 + x1 >= 2.0f * px) == from_p, up_y = (y0 + y1 >= 2.0f * py) == from_p,
+               up_z = (z0 + z1 >= 2.0f * pz) == from_p;
+    const float mrg = beam_margin(G, px, py, pz, x0, y0, z0, x1, y1, z1);
+    const BeamAxis x = beam_axis(px, x0 - px, x1 - px, mrg), y = beam_axis(py, y0 - py, y1 - py, mrg),
+                   z = beam_axis(pz, z0 - pz, z1 - pz, mrg);
+    const int nsub = 1 << (3 * (G.mshift - 2));
+    bool hit = false;
+    for (int i = 0; i < n; ++i) {
+        const uint2 w = list[i];
+        const int xy = __builtin_amdgcn_readfirstlane((int)w.x),
+                  jz = __builtin_amdgcn_readfirstlane((int)w.y);
+        const int jx = xy & 0xffff, jy = (int)((uint32_t)xy >> 16);
+        int cx, cy, cz;
+        unsigned long long subs = __ballot(
+            pencil_sub(G, x, y, z, jx, jy, jz, lane < nsub ? lane : 0, cx, cy, cz) && lane < nsub);
+        for (; subs != 0; subs &= subs - 1) {
+            const int s = (int)__builtin_ctzll(subs);
+            int32_t b, e;
+            pencil_cell(G, box, x, y, z, __builtin_amdgcn_readlane(cx, s),
+                        __builtin_amdgcn_readlane(cy, s), __builtin_amdgcn_readlane(cz, s), lane, up_x,
+                        up_y, up_z, b, e);
+            for (unsigned long long live = __ballot(b < e); live != 0; live &= live - 1) {
+                const int l = (int)__builtin_ctzll(live);
+                const int32_t j1 = __builtin_amdgcn_readlane(e, l);
+                for (int32_t j = __builtin_amdgcn_readlane(b, l); j < j1; ++j) {
+                    double tt;
+                    hit |= hit_numba(rt, rt.len, load_rec(recs, j), tt);
+                }
+                if (!__ballot(walk && !hit))
+                    return hit;
+            }
+        }
+    }
+    return hit && walk;
+}
+
 // Persistent form of k_visibility_grid: each workgroup copies the quantised
 // macro table (at most lds_table(WPC) blocks) into LDS once; then each
 // wavefront repeatedly claims a 64-ray word of output (one atomic on one of
 // the 8 counters next_task[0..7]), so waves never wait for one another and
 // the load balances whatever number of workgroups is resident.  Dead-block
-// tests read LDS.  WPC: workgroups per CU the registers are bounded for.  BEAM: the
-// words' rays walk as beams (lem_beam_walk.h) where their words allow it.
-template <bool ANY, bool SINK_MAJOR, int SEM, bool REV, int WPC, bool BEAM>
+// tests read LDS.  WPC: workgroups per CU the registers are bounded for.  WALK: the
+// words' rays walk one by one, or as beams or pencils (lem_beam_walk.h) where their
+// words allow it.
+template <bool ANY, bool SINK_MAJOR, int SEM, bool REV, int WPC, int WALK>
 __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
     const float *__restrict__ src, int64_t S, const float *__restrict__ snk, int64_t K, GridDev G,
     const int32_t *__restrict__ cell_start, const float4 *__restrict__ recs,
@@ -699,15 +762,12 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
     float *__restrict__ dist_out, unsigned long long *__restrict__ next_task, int skip_self,
     unsigned long long *__restrict__ par_count, uint2 *__restrict__ par_queue, int64_t par_cap,
     int perm, const int32_t *__restrict__ outer_order, const float *__restrict__ word_box,
-    const unsigned long long *__restrict__ narrow)
+    const unsigned long long *__restrict__ chosen)
 {
-    // both walks are launched where beams may serve; the words' boxes decide
-    if constexpr (!REV && SEM == LEM_SEM_NUMBA)
-        if (narrow) {
-            const int64_t words = ((SINK_MAJOR ? S : K) + 63) / 64;
-            if ((2 * (int64_t)*narrow >= words) != BEAM)
-                return;
-        }
+    // every walk is launched that may serve, and the words' boxes decide
+    constexpr bool BEAM = WALK != WALK_RAY;
+    if (chosen && (int)*chosen != WALK)
+        return;
     __shared__ uint2 s_list[BEAM ? GB / 64 * BEAM_WORDS : 1][BEAM_LIST];
     __shared__ uint32_t smqa[lds_table(WPC)];
     __shared__ uint16_t smqb[lds_table(WPC)];
@@ -783,6 +843,7 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
         const int64_t w0 = owner * CH + u * CLAIM_WORDS;
         const int64_t end = (int64_t)(owner + 1) * CH < W ? (int64_t)(owner + 1) * CH : W;
         const int64_t w1 = w0 + CLAIM_WORDS < end ? w0 + CLAIM_WORDS : end;
+        const float *P = SINK_MAJOR ? snk + 3 * outer : src + 3 * outer;
         // one word of 64 rays; n: blocks of its beam's list (-1: walk one by one)
         auto cast_word = [&](int64_t word, int n, const uint2 *list) {
             const int64_t slot = word * 64 + lane;
@@ -804,7 +865,8 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
             // queued for k_visibility_grid_par (left unblocked, at full
             // length, here), which keeps that walk's registers and code out
             // of this kernel
-            if (walk && (rw.dx == 0.0f || rw.dy == 0.0f || rw.dz == 0.0f)) {
+            if ((WALK != WALK_PENCIL || n < 0) && walk &&
+                (rw.dx == 0.0f || rw.dy == 0.0f || rw.dz == 0.0f)) {
                 walk = false;
                 // past the capacity the count only has to stay above it
                 if (__atomic_load_n(par_count, __ATOMIC_RELAXED) <= (unsigned long long)par_cap) {
@@ -813,7 +875,12 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
                         par_queue[q] = make_uint2((unsigned int)outer, (unsigned int)slot);
                 }
             }
-            if (BEAM && n >= 0) {
+            if (WALK == WALK_PENCIL && n >= 0) {
+                if constexpr (ANY && WALK == WALK_PENCIL)
+                    if (n > 0)
+                        hit = pencil_cast(walk, r, G, recs, box, word_box + 6 * word, P[0], P[1], P[2],
+                                          SINK_MAJOR == REV, list, n);
+            } else if (BEAM && n >= 0) {
                 // a source on its sink has no direction and meets nothing
                 if (n > 0)
                     hit = beam_cast<ANY, SEM>(walk && rw.len > 0.0f, rw, r, G, cell_start, recs, box,
@@ -839,7 +906,6 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
                 dist_out[outer * NI + inner] = dist;
         };
         if constexpr (BEAM) {
-            const float *P = SINK_MAJOR ? snk + 3 * outer : src + 3 * outer;
             uint2 (*list)[BEAM_LIST] = s_list + (threadIdx.x >> 6) * BEAM_WORDS;
             for (int64_t word = w0; word < w1; word += BEAM_WORDS) {
                 const int cnt = beam_lists(G, smq, word_box, word, w1, P[0], P[1], P[2],
@@ -857,11 +923,14 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
     }
 }
 
-// clears the 8 task counters of the persistent traversal and the count of narrow words
+// clears the 8 task counters of the persistent traversal and the two counts of narrow
+// words
 __global__ void k_zero_u64(unsigned long long *__restrict__ p)
 {
     if (threadIdx.x < 9)
         p[threadIdx.x * COUNTER_STRIDE] = 0ull;
+    else if (threadIdx.x == 9)
+        p[8 * COUNTER_STRIDE + 1] = 0ull;
 }
 
 __global__ __launch_bounds__(GB) void k_zero_words(unsigned long long *__restrict__ p, int64_t n)
@@ -1532,22 +1601,26 @@ extern "C" int lem_visibility_grid(const float *src, int64_t S, const float *snk
         const int64_t nwg =
             std::max<int64_t>(1, std::min<int64_t>(ceil_div(words, 4), (int64_t)cus * per_cu));
         hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, L.counter);
-        // Beams serve rays in a spatial order whose words are narrow (k_word_boxes) and
-        // that go on past the first blocks: not those walked from the sink end, whose
-        // hits are near it (5,000 to 50,000 triangles, 3,600 sources x 30,000 sinks:
-        // 3.37 and 5.74 ms one by one, 3.43 and 6.03 as beams).  BEAM_NARROW: the same
-        // triangles, 30,000 sources to a plate of 33 x 33 sinks, 2.5 and 11 square
-        // blocks a word, 2.56 and 7.45 ms one by one, 2.91 and 8.65 as beams; terrain of
-        // 10^6 triangles, 512 sinks, words of 0.08, 0.3, 1.3 and 5 square blocks: 37.1,
-        // 14.4, 7.4 and 6.0 -> 21.7, 9.8, 5.5 and 4.9.  Below 2^22 rays the boxes and
-        // the launch are not worth it.  The boxes take the place of the Morton keys.
+        // Beams and pencils serve rays in a spatial order whose words are narrow.
+        // Pencils, any hit: 5,000 and 50,000 triangles, 3,600 sources within a tenth of
+        // a cell x 30,000 sinks, 5.25 and 9.95 ms one by one -> 3.17 and 7.02 (from the
+        // sink end 3.37 and 5.74 -> 2.57 and 4.70).  Beams, for rays that go on past the
+        // first blocks (from the sink end the same calls took 3.43 and 6.03 as beams): a
+        // terrain of 10^6 triangles, 512 sinks, words of 0.08, 0.3, 1.3 and 5 square
+        // blocks: 37.1, 14.4, 7.4 and 6.0 -> 21.7, 9.8, 5.5 and 4.9; but 30,000 sources
+        // among those triangles to a plate of 33 x 33 sinks, 2.5 and 11 square blocks a
+        // word: 2.56 and 7.45 -> 2.91 and 8.65.  Below 2^22 rays the boxes and the
+        // launches are not worth it.  The boxes take the place of the Morton keys.
         float *word_box = nullptr;
-        unsigned long long *narrow = nullptr;
-        if (order && !rev && semantics != LEM_SEM_NATIVE && (double)S * (double)K >= 4194304.0) {
+        unsigned long long *chosen = nullptr;
+        if (order && semantics != LEM_SEM_NATIVE && (double)S * (double)K >= 4194304.0) {
             word_box = reinterpret_cast<float *>(L.k0);
-            narrow = L.counter + 8 * COUNTER_STRIDE;
+            unsigned long long *narrow = L.counter + 8 * COUNTER_STRIDE;
+            chosen = narrow + 2;
             hipLaunchKernelGGL(k_word_boxes, dim3((unsigned)nbl), dim3(GB), 0, st,
                                sink_major ? src : snk, NI, order, G, word_box, narrow);
+            hipLaunchKernelGGL(k_choose_walk, dim3(1), dim3(64), 0, st, narrow, Wn, any ? 1 : 0,
+                               rev ? 1 : 0, chosen);
         }
         const int64_t nbeam =
             std::max<int64_t>(1, std::min<int64_t>(ceil_div(words, 4), (int64_t)cus * BEAM_WPC));
@@ -1557,20 +1630,20 @@ extern "C" int lem_visibility_grid(const float *src, int64_t S, const float *snk
         unsigned long long *pcount = reinterpret_cast<unsigned long long *>(qb);
         uint2 *pq = reinterpret_cast<uint2 *>(qb + 256);
         hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(GB), 0, st, pcount, 1);
+#define LEM_WALK(A, M, SM, R, WP, WALK, NWG)                                                  \
+    hipLaunchKernelGGL((k_visibility_grid_lds<A, M, SM, R, WP, WALK>), dim3((unsigned)(NWG)), \
+                       dim3(GB), 0, st, src, S, snk, K, G, cell_start, rc4, bx4, mq,          \
+                       info->nmacro, order, hb, dist, L.counter, skip_self, pcount, pq,       \
+                       PAR_QUEUE_CAP, perm ? 1 : 0, outer_order, word_box, chosen)
 #define LEM_VGL(A, M, SM, R, WP)                                                              \
     do {                                                                                      \
-        if constexpr (!R && SM == LEM_SEM_NUMBA) {                                            \
+        if constexpr (A && SM == LEM_SEM_NUMBA)                                               \
             if (word_box)                                                                     \
-                hipLaunchKernelGGL((k_visibility_grid_lds<A, M, SM, R, BEAM_WPC, true>),      \
-                                   dim3((unsigned)nbeam), dim3(GB), 0, st, src, S, snk, K, G, \
-                                   cell_start, rc4, bx4, mq, info->nmacro, order, hb, dist,   \
-                                   L.counter, skip_self, pcount, pq, PAR_QUEUE_CAP, perm ? 1 : 0, \
-                                   outer_order, word_box, narrow);                            \
-        }                                                                                     \
-        hipLaunchKernelGGL((k_visibility_grid_lds<A, M, SM, R, WP, false>), dim3((unsigned)nwg), \
-                           dim3(GB), 0, st, src, S, snk, K, G, cell_start, rc4, bx4, mq,      \
-                           info->nmacro, order, hb, dist, L.counter, skip_self, pcount, pq,   \
-                           PAR_QUEUE_CAP, perm ? 1 : 0, outer_order, nullptr, narrow);        \
+                LEM_WALK(A, M, SM, R, BEAM_WPC, WALK_PENCIL, nbeam);                          \
+        if constexpr (!R && SM == LEM_SEM_NUMBA)                                              \
+            if (word_box)                                                                     \
+                LEM_WALK(A, M, SM, R, BEAM_WPC, WALK_BEAM, nbeam);                            \
+        LEM_WALK(A, M, SM, R, WP, WALK_RAY, nwg);                                             \
         hipLaunchKernelGGL((k_visibility_grid_par<A, M, SM, R>), dim3((unsigned)nwg), dim3(GB), 0, \
                            st, src, S, snk, K, G, cell_start, rc4, bx4, mq, info->nmacro, order, \
                            hb, dist, skip_self, pcount, pq, PAR_QUEUE_CAP, perm ? 1 : 0);      \
@@ -1601,6 +1674,7 @@ extern "C" int lem_visibility_grid(const float *src, int64_t S, const float *snk
         }
 #undef LEM_VGL2
 #undef LEM_VGL
+#undef LEM_WALK
         int rc = check_launch("k_visibility_grid_lds / k_visibility_grid_par");
         if (rc || !perm)
             return rc;

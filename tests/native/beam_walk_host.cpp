@@ -75,6 +75,62 @@ bool beam_host(const HostGrid &H, const float *P, const std::vector<const float 
     return true;
 }
 
+// One wavefront as a pencil, any hit; the lanes' hits.
+bool pencil_host(const HostGrid &H, const float *P, const std::vector<const float *> &Q, bool from_p,
+                 const std::vector<Ray> &rt, std::vector<char> &hit)
+{
+    const GridDev &G = H.G;
+    const MacroTab smq{H.qa.data(), H.qb.data(), H.axis};
+    float lo[3], hi[3];
+    for (int a = 0; a < 3; ++a) {
+        lo[a] = hi[a] = Q[0][a];
+        for (auto q : Q) {
+            lo[a] = fminf(lo[a], q[a]);
+            hi[a] = fmaxf(hi[a], q[a]);
+        }
+    }
+    Beam b;
+    if (!beam_of(G, P[0], P[1], P[2], lo[0], lo[1], lo[2], hi[0], hi[1], hi[2], from_p, b))
+        return false;
+    BeamAxis ax[3];
+    bool up[3];
+    const float mrg = beam_margin(G, P[0], P[1], P[2], lo[0], lo[1], lo[2], hi[0], hi[1], hi[2]);
+    for (int a = 0; a < 3; ++a) {
+        ax[a] = beam_axis(P[a], lo[a] - P[a], hi[a] - P[a], mrg);
+        up[a] = (lo[a] + hi[a] >= 2.0f * P[a]) == from_p;
+    }
+    hit.assign(Q.size(), 0);
+    for (int s = 0; s < b.slabs; ++s) {
+        const int j = b.first + b.step * s;
+        int a0, na, b0, nb;
+        const int cnt = beam_slab(b, j, a0, na, b0, nb);
+        if (cnt > BEAM_MAX || (cnt > 0 && (na > BEAM_NA || nb > BEAM_NB)))
+            return false;
+        for (uint32_t m = cnt ? beam_mask(G, smq, b.axis, ax[0], ax[1], ax[2], j, a0, na, b0, cnt) : 0;
+             m; m &= m - 1) {
+            const int bit = __builtin_ctz(m);
+            int jx, jy, jz;
+            beam_block_at(b.axis, j, a0 + (bit & 7), b0 + (bit >> 3), jx, jy, jz);
+            for (int sub = 0; sub < 1 << (3 * (G.mshift - 2)); ++sub) {
+                int cx, cy, cz;
+                if (!pencil_sub(G, ax[0], ax[1], ax[2], jx, jy, jz, sub, cx, cy, cz))
+                    continue;
+                for (int l = 0; l < 64; ++l) {
+                    int32_t r0, r1;
+                    pencil_cell(G, H.box.data(), ax[0], ax[1], ax[2], cx, cy, cz, l, up[0], up[1],
+                                up[2], r0, r1);
+                    for (int32_t r = r0; r < r1; ++r)
+                        for (size_t i = 0; i < Q.size(); ++i) {
+                            double tt;
+                            hit[i] |= hit_numba(rt[i], rt[i].len, load_rec(H.recs.data(), r), tt);
+                        }
+                }
+            }
+        }
+    }
+    return true;
+}
+
 int64_t g_beams = 0, g_refused = 0;
 
 // clusters of 64 around points of `centres`, radii of `frac` of the scene and less
@@ -147,6 +203,13 @@ void check_beams(Scene sc, float cells_per_tri, int force_mshift, uint64_t seed)
                         : mode <= 2 ? beam_host<true, 0>(H, P, Q, from_p, r, rt, walk, h)
                                     : beam_host<true, 1>(H, P, Q, from_p, r, rt, walk, h);
                     ++beams;
+                    if ((mode == 1 || mode == 2) && H.info.mshift >= 2 && H.info.mshift <= 4) {
+                        std::vector<char> p;
+                        if (pencil_host(H, P, Q, from_p, rt, p) != ok)
+                            ++bad;
+                        for (int i = 0; ok && i < 64; ++i)
+                            bad += p[i] != hit[back ? k * S + s0 + i : (s0 + i) * K + k];
+                    }
                     if (!ok) {
                         ++refused;
                         continue;

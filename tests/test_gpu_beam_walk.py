@@ -27,13 +27,16 @@ def _points(rng, kind, n):
     elif kind == "clusters":
         c = rng.uniform([0, 0, -1], [40, 40, 6], (n // 64 + 1, 3))
         p = (np.repeat(c, 64, 0) + rng.normal(size=(64 * (n // 64 + 1), 3)) * 0.05)[:n]
+    elif kind == "pencil":  # all within a fraction of a cell
+        p = rng.normal(size=(n, 3)) * 0.02 + [20.0, 20.0, 4.0]
+        p[:n // 2, 2] = 4.0
     else:                   # far origins
         p = rng.normal(size=(n, 3)) * 5 + [2000.0, -1500.0, 900.0]
     return p.astype(np.float32)
 
 
 @pytest.mark.parametrize("kind,n", [("grid", 8191), ("grid", 65536), ("clusters", 20000),
-                                    ("far", 12345)])
+                                    ("far", 12345), ("pencil", 8000)])
 @pytest.mark.parametrize("sink_major", [True, False])
 def test_beams_equal_the_dense_masks(native, kind, n, sink_major):
     rng = np.random.default_rng(n)
