@@ -548,6 +548,7 @@ constexpr int COUNTER_STRIDE = 512;  // uint64 elements
 // 3 / 8 / 12 / 16 / 32 words gave C2 (1M-triangle terrain) 1,105 / 1,084 /
 // 1,083 / 1,089 / 1,093 ms and C3 (one bounce) 758 / 738 / 736 / 733 / 732 ms.
 constexpr int CLAIM_WORDS = 12;
+constexpr int CLAIM_DEPTH = 8;  // claims for each resident wavefront, before they are longer than a word
 
 // Box of the points of each word of 64 lane slots: box[word] = lo, hi; counts the
 // narrow ones, whose two longest sides span at most BEAM_NARROW square macro blocks
@@ -587,12 +588,12 @@ __global__ __launch_bounds__(GB) void k_word_boxes(const float *__restrict__ p, 
 
 // The walk of a call, from its words: chosen = WALK_*.
 __global__ void k_choose_walk(const unsigned long long *__restrict__ narrow, int64_t words, int any,
-                              int rev, unsigned long long *__restrict__ chosen)
+                              int beams, unsigned long long *__restrict__ chosen)
 {
     if (threadIdx.x == 0)
-        *chosen = any && 2 * (int64_t)narrow[1] >= words    ? WALK_PENCIL
-                  : !rev && 2 * (int64_t)narrow[0] >= words ? WALK_BEAM
-                                                            : WALK_RAY;
+        *chosen = any && 2 * (int64_t)narrow[1] >= words     ? WALK_PENCIL
+                  : beams && 2 * (int64_t)narrow[0] >= words ? WALK_BEAM
+                                                             : WALK_RAY;
 }
 
 constexpr int BEAM_WORDS = 4;  // words whose beams a wavefront finds at once, 16 lanes each
@@ -761,8 +762,8 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
     const int32_t *__restrict__ order, unsigned long long *__restrict__ bits,
     float *__restrict__ dist_out, unsigned long long *__restrict__ next_task, int skip_self,
     unsigned long long *__restrict__ par_count, uint2 *__restrict__ par_queue, int64_t par_cap,
-    int perm, const int32_t *__restrict__ outer_order, const float *__restrict__ word_box,
-    const unsigned long long *__restrict__ chosen)
+    int perm, int claim, const int32_t *__restrict__ outer_order,
+    const float *__restrict__ word_box, const unsigned long long *__restrict__ chosen)
 {
     // every walk is launched that may serve, and the words' boxes decide
     constexpr bool BEAM = WALK != WALK_RAY;
@@ -790,8 +791,8 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
     // counter, so its L2 holds the cells of one region; an XCD whose share is
     // done claims from the next counters.
     const int64_t CH = (W + 7) / 8;
-    // a claim takes CLAIM_WORDS consecutive words of the owner's eighth
-    const int64_t UPR = (CH + CLAIM_WORDS - 1) / CLAIM_WORDS;
+    // a claim takes `claim` consecutive words of the owner's eighth
+    const int64_t UPR = (CH + claim - 1) / claim;
     int owner = (int)(blockIdx.x & 7), tried = 0;
     for (;;) {
         unsigned long long t = 0;
@@ -840,9 +841,9 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
         // claims walk the outer points in a spatial order (consecutive claims
         // share cells in L2); rows are written at the point's own index
         const int64_t outer = outer_order ? (int64_t)outer_order[oc] : oc;
-        const int64_t w0 = owner * CH + u * CLAIM_WORDS;
+        const int64_t w0 = owner * CH + u * claim;
         const int64_t end = (int64_t)(owner + 1) * CH < W ? (int64_t)(owner + 1) * CH : W;
-        const int64_t w1 = w0 + CLAIM_WORDS < end ? w0 + CLAIM_WORDS : end;
+        const int64_t w1 = w0 + claim < end ? w0 + claim : end;
         const float *P = SINK_MAJOR ? snk + 3 * outer : src + 3 * outer;
         // one word of 64 rays; n: blocks of its beam's list (-1: walk one by one)
         auto cast_word = [&](int64_t word, int n, const uint2 *list) {
@@ -1600,27 +1601,35 @@ extern "C" int lem_visibility_grid(const float *src, int64_t S, const float *snk
         const int64_t words = NO * ceil_div(NI, 64);
         const int64_t nwg =
             std::max<int64_t>(1, std::min<int64_t>(ceil_div(words, 4), (int64_t)cus * per_cu));
+        // Few words: short claims, or most of the resident wavefronts get none while
+        // the others walk one word behind the other (a terrain of 10^6 triangles, 4,096
+        // words of 64 x 64 sources and 64 sinks: 4.0 ms in claims of 12, 1.06 of 1;
+        // 65,536 words: 6.0 -> 2.0).
+        const int claim =
+            (int)std::max<int64_t>(1, std::min<int64_t>(CLAIM_WORDS, words / (nwg * 4 * CLAIM_DEPTH)));
         hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, L.counter);
         // Beams and pencils serve rays in a spatial order whose words are narrow.
         // Pencils, any hit: 5,000 and 50,000 triangles, 3,600 sources within a tenth of
         // a cell x 30,000 sinks, 5.25 and 9.95 ms one by one -> 3.17 and 7.02 (from the
-        // sink end 3.37 and 5.74 -> 2.57 and 4.70).  Beams, for rays that go on past the
-        // first blocks (from the sink end the same calls took 3.43 and 6.03 as beams): a
-        // terrain of 10^6 triangles, 512 sinks, words of 0.08, 0.3, 1.3 and 5 square
+        // sink end 3.37 and 5.74 -> 2.57 and 4.70).  Beams, for rays that meet in P: those
+        // that start there may all end in the first blocks, while the list goes on (from
+        // a scatterer, three in four blocked: the same calls 3.43 and 6.03 as beams, the
+        // legs of 200,000 scatterers to a fine shell 143 -> 162).  A terrain of 10^6
+        // triangles, 512 sinks, words of 0.08, 0.3, 1.3 and 5 square
         // blocks: 37.1, 14.4, 7.4 and 6.0 -> 21.7, 9.8, 5.5 and 4.9; but 30,000 sources
         // among those triangles to a plate of 33 x 33 sinks, 2.5 and 11 square blocks a
-        // word: 2.56 and 7.45 -> 2.91 and 8.65.  Below 2^22 rays the boxes and the
+        // word: 2.56 and 7.45 -> 2.91 and 8.65.  Below 2^18 rays the boxes and the
         // launches are not worth it.  The boxes take the place of the Morton keys.
         float *word_box = nullptr;
         unsigned long long *chosen = nullptr;
-        if (order && semantics != LEM_SEM_NATIVE && (double)S * (double)K >= 4194304.0) {
+        if (order && semantics != LEM_SEM_NATIVE && (double)S * (double)K >= 262144.0) {
             word_box = reinterpret_cast<float *>(L.k0);
             unsigned long long *narrow = L.counter + 8 * COUNTER_STRIDE;
             chosen = narrow + 2;
             hipLaunchKernelGGL(k_word_boxes, dim3((unsigned)nbl), dim3(GB), 0, st,
                                sink_major ? src : snk, NI, order, G, word_box, narrow);
             hipLaunchKernelGGL(k_choose_walk, dim3(1), dim3(64), 0, st, narrow, Wn, any ? 1 : 0,
-                               rev ? 1 : 0, chosen);
+                               sink_major && !rev ? 1 : 0, chosen);
         }
         const int64_t nbeam =
             std::max<int64_t>(1, std::min<int64_t>(ceil_div(words, 4), (int64_t)cus * BEAM_WPC));
@@ -1634,13 +1643,13 @@ extern "C" int lem_visibility_grid(const float *src, int64_t S, const float *snk
     hipLaunchKernelGGL((k_visibility_grid_lds<A, M, SM, R, WP, WALK>), dim3((unsigned)(NWG)), \
                        dim3(GB), 0, st, src, S, snk, K, G, cell_start, rc4, bx4, mq,          \
                        info->nmacro, order, hb, dist, L.counter, skip_self, pcount, pq,       \
-                       PAR_QUEUE_CAP, perm ? 1 : 0, outer_order, word_box, chosen)
+                       PAR_QUEUE_CAP, perm ? 1 : 0, claim, outer_order, word_box, chosen)
 #define LEM_VGL(A, M, SM, R, WP)                                                              \
     do {                                                                                      \
         if constexpr (A && SM == LEM_SEM_NUMBA)                                               \
             if (word_box)                                                                     \
                 LEM_WALK(A, M, SM, R, BEAM_WPC, WALK_PENCIL, nbeam);                          \
-        if constexpr (!R && SM == LEM_SEM_NUMBA)                                              \
+        if constexpr (M && !R && SM == LEM_SEM_NUMBA)                                         \
             if (word_box)                                                                     \
                 LEM_WALK(A, M, SM, R, BEAM_WPC, WALK_BEAM, nbeam);                            \
         LEM_WALK(A, M, SM, R, WP, WALK_RAY, nwg);                                             \
