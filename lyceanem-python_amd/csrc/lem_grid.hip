@@ -889,7 +889,10 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
             } else if (walk) {
                 float dw = rw.len;
                 float &dd = REV ? dw : dist;
-                hit = dda_cast<ANY, SEM, true, false>(rw, dd, G, cell_start, recs, box, nullptr,
+                if constexpr (!ANY)
+                    hit = closest_cast(r, dist, G, cell_start, recs, box, smq);
+                else
+                    hit = dda_cast<ANY, SEM, true, false>(rw, dd, G, cell_start, recs, box, nullptr,
                                                       nullptr, nullptr, smq, REV ? &r : nullptr);
             }
             if (order && !perm) {

@@ -203,6 +203,16 @@ void check_beams(Scene sc, float cells_per_tri, int force_mshift, uint64_t seed)
                         : mode <= 2 ? beam_host<true, 0>(H, P, Q, from_p, r, rt, walk, h)
                                     : beam_host<true, 1>(H, P, Q, from_p, r, rt, walk, h);
                     ++beams;
+                    if (mode == 0)  // the same rays one by one, blocks skipped in a loop of their own
+                        for (int i = 0; i < 64; ++i)
+                            if (walk[i]) {
+                                const int64_t at = back ? k * S + s0 + i : (s0 + i) * K + k;
+                                float d = r[i].len;
+                                const bool hc = closest_cast(
+                                    r[i], d, H.G, H.cell_start.data(), H.recs.data(), H.box.data(),
+                                    MacroTab{H.qa.data(), H.qb.data(), H.axis});
+                                bad += hc != hit[at] || std::memcmp(&d, &dist[at], 4) != 0;
+                            }
                     if ((mode == 1 || mode == 2) && H.info.mshift >= 2 && H.info.mshift <= 4) {
                         std::vector<char> p;
                         if (pencil_host(H, P, Q, from_p, rt, p) != ok)
