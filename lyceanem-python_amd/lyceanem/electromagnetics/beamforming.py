@@ -13,7 +13,6 @@ import contextvars
 from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
-import torch
 
 from .. import _native
 
@@ -107,6 +106,8 @@ def _in_row_blocks(work, n, width):
     element is computed by the same numpy operations however the rows are cut.
     2,701 commands x 256 elements: 73 ms in one piece, 9.5 in 16 threads;
     1,891 x 81: 15.0, 4.4 (in 9; 5.8 in 16, which wait for each other too often)."""
+    import torch
+
     threads = max(1, min(torch.get_num_threads(), n * width // _BLOCK_MIN))
     rounds = -(-n * width // (threads * _BLOCK_MAX))
     step = max(1, -(-n // max(threads * rounds, 1)))
