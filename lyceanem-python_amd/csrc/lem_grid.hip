@@ -703,7 +703,9 @@ LEM_DEV bool beam_cast(bool walk, const Ray &r, const Ray &rt, const GridDev &G,
 // As beam_cast for a pencil, any hit: the word's cells and their triangles are the same
 // for all its rays, so triangles come through scalar loads and every lane tests each.
 // 50,000 triangles, 3,600 sources x 30,001 sinks from the sink end: 5.74 ms one by one,
-// 2,615 vector instructions and 81 vector loads a word; 4.70 ms, 1,663 and 29.
+// 2,615 vector instructions and 81 vector loads a word; 4.47 ms, 1,500 and 29.
+// (Measured and left: the next triangle loaded before this one is tested, 1 % slower;
+// four workgroups a CU without spills, 3 %.)
 LEM_DEV bool pencil_cast(bool walk, const Ray &rt, const GridDev &G, const float4 *__restrict__ recs,
                          const float4 *__restrict__ box, const float *__restrict__ wb, float px,
                          float py, float pz, bool from_p, const uint2 *list, int n)
@@ -722,15 +724,22 @@ LEM_DEV bool pencil_cast(bool walk, const Ray &rt, const GridDev &G, const float
         const int xy = __builtin_amdgcn_readfirstlane((int)w.x),
                   jz = __builtin_amdgcn_readfirstlane((int)w.y);
         const int jx = xy & 0xffff, jy = (int)((uint32_t)xy >> 16);
-        int cx, cy, cz;
-        unsigned long long subs = __ballot(
-            pencil_sub(G, x, y, z, jx, jy, jz, lane < nsub ? lane : 0, cx, cy, cz) && lane < nsub);
+        // a block of 4 x 4 x 4 cells is its own sub-block, and known to be met
+        int cx = jx << 2, cy = jy << 2, cz = jz << 2;
+        unsigned long long subs = 1;
+        if (nsub > 1)
+            subs = __ballot(
+                pencil_sub(G, x, y, z, jx, jy, jz, lane < nsub ? lane : 0, cx, cy, cz) && lane < nsub);
         for (; subs != 0; subs &= subs - 1) {
-            const int s = (int)__builtin_ctzll(subs);
+            int sx = cx, sy = cy, sz = cz;
+            if (nsub > 1) {
+                const int s = (int)__builtin_ctzll(subs);
+                sx = __builtin_amdgcn_readlane(cx, s);
+                sy = __builtin_amdgcn_readlane(cy, s);
+                sz = __builtin_amdgcn_readlane(cz, s);
+            }
             int32_t b, e;
-            pencil_cell(G, box, x, y, z, __builtin_amdgcn_readlane(cx, s),
-                        __builtin_amdgcn_readlane(cy, s), __builtin_amdgcn_readlane(cz, s), lane, up_x,
-                        up_y, up_z, b, e);
+            pencil_cell(G, box, x, y, z, sx, sy, sz, lane, up_x, up_y, up_z, b, e);
             for (unsigned long long live = __ballot(b < e); live != 0; live &= live - 1) {
                 const int l = (int)__builtin_ctzll(live);
                 const int32_t j1 = __builtin_amdgcn_readlane(e, l);
@@ -1613,8 +1622,8 @@ extern "C" int lem_visibility_grid(const float *src, int64_t S, const float *snk
         hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, L.counter);
         // Beams and pencils serve rays in a spatial order whose words are narrow.
         // Pencils, any hit: 5,000 and 50,000 triangles, 3,600 sources within a tenth of
-        // a cell x 30,000 sinks, 5.25 and 9.95 ms one by one -> 3.17 and 7.02 (from the
-        // sink end 3.37 and 5.74 -> 2.57 and 4.70).  Beams, for rays that meet in P: those
+        // a cell x 30,000 sinks, 5.25 and 9.95 ms one by one -> 2.85 and 6.66 (from the
+        // sink end 3.37 and 5.74 -> 2.37 and 4.47).  Beams, for rays that meet in P: those
         // that start there may all end in the first blocks, while the list goes on (from
         // a scatterer, three in four blocked: the same calls 3.43 and 6.03 as beams, the
         // legs of 200,000 scatterers to a fine shell 143 -> 162).  A terrain of 10^6
