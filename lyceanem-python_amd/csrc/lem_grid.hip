@@ -747,8 +747,9 @@ LEM_DEV bool pencil_cast(bool walk, const Ray &rt, const GridDev &G, const float
                     double tt;
                     hit |= hit_numba(rt, rt.len, load_rec(recs, j), tt);
                 }
+                // lanes without a ray of their own test along and may hit
                 if (!__ballot(walk && !hit))
-                    return hit;
+                    return hit && walk;
             }
         }
     }
