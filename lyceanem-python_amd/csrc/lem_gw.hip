@@ -12,22 +12,27 @@
 // wavenumber k_f, d = (p_k - p_s)/r and a fixed source polarisation e.
 //
 // FP32 matrix instructions run at 1/16 of the bfloat16 rate, so both factors are
-// split into three bfloat16 parts, x = x1 + x2 + x3 exactly (8 bits of the
-// significand each, by truncation: full float32 range, no scaling), and the six
-// products x1 y1, x1 y2, x2 y1, x2 y2, x1 y3, x3 y1 accumulate in float32 with
-// v_mfma_f32_32x32x16_bf16; the three left out are below 2^-24 of x y.  A step of
-// 16 sources is summed from zero and added to the running sums with ordinary
-// float32 additions.  Error against float64, 4,096 sources: 3e-7 (the FP32
-// instructions' chain of 4,096 roundings: 1.6e-6).
+// split into three bfloat16 parts, x = x1 + x2 + x3 exactly (x1 and x2 rounded to
+// nearest: |x2| <= 2^-8, |x3| <= 2^-17 for 1 <= |x| < 2; full float32 range, no
+// scaling), and the six products x1 y1, x1 y2, x2 y1, x2 y2, x1 y3, x3 y1 accumulate in
+// float32 with v_mfma_f32_32x32x16_bf16; the three left out are at most 2^-24 of x y
+// together and of either sign.  The matrix instructions' own accumulation does not
+// round to nearest, so the five small products have sums of their own and a step of 16
+// sources is added up with ordinary float32 additions (gw_products).
+// Errors, in brackets those of FP32 instructions: of one source's products against
+// float64, 2.6e-8 (3.1e-8; parts cut off instead of rounded, in one chain: 7.0e-8 and
+// always towards zero); of the sum of 1 / 16 / 1,024 sources, G included, 1.60e-7 /
+// 1.90e-7 / 2.03e-7 (1.61e-7 / 2.08e-7 / 8.2e-7).
 //
 // Per step 72 matrix instructions (2,304 cycles) multiply a tile of 32 sinks x 32
 // sets x 3 components, and preparing it takes about 500 vector instructions: what
 // bounds both kernels below is that the two only overlap between wavefronts of a
-// SIMD, of which the 96 sums and 32 partial ones leave room for two.  64 x 64
-// sources, 16,384 sinks, 16 frequencies: 13.87 ms (FP32 instructions) -> 8.25 ms;
-// 32 x 32 sources, 2,720 sinks, one frequency: 186 -> 78 us.  (Measured and
+// SIMD, of which the 96 sums and 48 partial ones leave room for two.  64 x 64
+// sources, 16,384 sinks, 16 frequencies: 13.87 ms (FP32 instructions) -> 8.78 ms;
+// 32 x 32 sources, 2,720 sinks, one frequency: 186 -> 73 us.  (Measured and
 // left: pairs of wavefronts that share G in LDS, 9.3 ms and 98 us; matrix and vector
-// instructions interleaved in one wavefront, 12 ms and more, with registers spilled.)
+// instructions interleaved in one wavefront, 12 ms and more, with registers spilled;
+// all six products in one chain, 8.48 ms and 74 us with an error of 3.4e-8.)
 #include "lem_device.h"
 #include "lem_internal.h"
 #include "../../include/lem.h"
@@ -36,6 +41,8 @@ namespace lem {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int GW_M = 32;    // sinks per wavefront
@@ -84,21 +91,22 @@ struct Planes {
 };
 
 LEM_DEV uint32_t bits_of(float x) { return __builtin_bit_cast(uint32_t, x); }
-LEM_DEV float head_of(float x) { return __builtin_bit_cast(float, bits_of(x) & 0xffff0000u); }
-// the upper halves of a and b in one word (a in the low half)
-LEM_DEV uint32_t upper_halves(float a, float b)
+// a and b rounded to bfloat16, in one word (a in the low half)
+LEM_DEV uint32_t rounded_pair(float a, float b)
 {
-    return __builtin_amdgcn_perm(bits_of(b), bits_of(a), 0x07060302u);
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
 }
+LEM_DEV float low_of(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
+LEM_DEV float high_of(uint32_t w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
 
-// the three parts of a and b, packed
+// the three parts of a and b, packed; the third are what is left, 8 bits at most
 LEM_DEV void split3(float a, float b, uint32_t &w0, uint32_t &w1, uint32_t &w2)
 {
-    const float a2 = a - head_of(a), b2 = b - head_of(b);
-    const float a3 = a2 - head_of(a2), b3 = b2 - head_of(b2);
-    w0 = upper_halves(a, b);
-    w1 = upper_halves(a2, b2);
-    w2 = upper_halves(a3, b3);
+    w0 = rounded_pair(a, b);
+    const float a2 = a - low_of(w0), b2 = b - high_of(w0);
+    w1 = rounded_pair(a2, b2);
+    const float a3 = a2 - low_of(w1), b3 = b2 - high_of(w1);
+    w2 = __builtin_amdgcn_perm(bits_of(b3), bits_of(a3), 0x07060302u);
 }
 
 LEM_DEV f32x16 mma(const bf16x8 &a, const bf16x8 &b, const f32x16 &c)
@@ -106,24 +114,35 @@ LEM_DEV f32x16 mma(const bf16x8 &a, const bf16x8 &b, const f32x16 &c)
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-// One component's 24 products, the smallest first: r = gr wr - gi wi, i = gr wi +
-// gi wr.  They start from zero and the step's sums are added with ordinary
-// additions: the matrix instructions' own accumulation does not round to nearest
-// (chained over 4,096 sources it left an error of 1.2e-5).
+// One component's 24 products: r = gr wr - gi wi, i = gr wi + gi wr.  They start from
+// zero and are added with ordinary additions: the matrix instructions' own accumulation
+// does not round to nearest (chained over 4,096 sources it left an error of 1.2e-5).
+// The large products x1 y1 stand apart from the small ones, the smallest of which come
+// first, so that a product is cut at its own last place once; one pair of them at a
+// time, for the registers (both at once, or the sums of two components pending in
+// k_gw_tile, spill up to 36: 11 to 12.6 ms instead of 8.78).
 LEM_DEV void gw_products(const Planes &gr, const Planes &gi, const Planes &wr, const Planes &wi,
                          const Planes &nwi, f32x16 &r, f32x16 &i)
 {
-    constexpr int A[6] = {0, 2, 1, 0, 1, 0}, B[6] = {2, 0, 1, 1, 0, 0};
+    constexpr int A[5] = {0, 2, 1, 0, 1}, B[5] = {2, 0, 1, 1, 0};
     const f32x16 zero = {};
     r = zero;
     i = zero;
 #pragma unroll
-    for (int q = 0; q < 6; ++q) {
+    for (int q = 0; q < 5; ++q) {
         r = mma(gr.h[A[q]], wr.h[B[q]], r);
         i = mma(gr.h[A[q]], wi.h[B[q]], i);
         r = mma(gi.h[A[q]], nwi.h[B[q]], r);
         i = mma(gi.h[A[q]], wr.h[B[q]], i);
     }
+    __builtin_amdgcn_sched_barrier(0);
+    f32x16 large = mma(gr.h[0], wr.h[0], zero);
+    large = mma(gi.h[0], nwi.h[0], large);
+    r += large;
+    __builtin_amdgcn_sched_barrier(0);
+    large = mma(gr.h[0], wi.h[0], zero);
+    large = mma(gi.h[0], wr.h[0], large);
+    i += large;
 }
 
 LEM_DEV bf16x8 flipped(const bf16x8 &x)
@@ -305,23 +324,23 @@ __global__ __launch_bounds__(512, 2) void k_gw_tile(
         for (int h = 0; h < 3; ++h)
             nwi.h[h] = flipped(wi.h[h]);
         Planes ar, ai;
-        f32x16 r0, i0, r1, i1;
+        f32x16 r, i;
         read_g(ar, ai, g, 1);
-        gw_products(gr, gi, wr, wi, nwi, r0, i0);
+        gw_products(gr, gi, wr, wi, nwi, r, i);
+        re[0] += r;
+        im[0] += i;
         read_g(gr, gi, g, 2);
-        gw_products(ar, ai, wr, wi, nwi, r1, i1);
-        re[0] += r0;
-        im[0] += i0;
+        gw_products(ar, ai, wr, wi, nwi, r, i);
+        re[1] += r;
+        im[1] += i;
         // every read of this buffer is done: the next step's operands are there
         __syncthreads();
         Planes nr, ni;
         read_w(nr, ni, s_w[(t + 1) & 1]);
         read_g(ar, ai, s_g[(t + 1) & 1], 0);
-        gw_products(gr, gi, wr, wi, nwi, r0, i0);
-        re[1] += r1;
-        im[1] += i1;
-        re[2] += r0;
-        im[2] += i0;
+        gw_products(gr, gi, wr, wi, nwi, r, i);
+        re[2] += r;
+        im[2] += i;
         wr = nr;
         wi = ni;
         gr = ar;
