@@ -552,9 +552,8 @@ constexpr int CLAIM_DEPTH = 8;  // claims for each resident wavefront, before th
 
 // Box of the points of each word of 64 lane slots: box[word] = lo, hi; counts the
 // narrow ones, whose two longest sides span at most BEAM_NARROW square macro blocks
-// (narrow[0]), and the pencils, at most BEAM_PENCIL square cells (narrow[1]).  One
-// wavefront a word.
-constexpr float BEAM_NARROW = 2.0f, BEAM_PENCIL = 0.25f;
+// (narrow[0]), and the pencils (narrow[1]).  One wavefront a word.
+constexpr float BEAM_NARROW = 2.0f;
 __global__ __launch_bounds__(GB) void k_word_boxes(const float *__restrict__ p, int64_t n,
                                                    const int32_t *__restrict__ order, GridDev G,
                                                    float *__restrict__ box,
@@ -574,24 +573,26 @@ __global__ __launch_bounds__(GB) void k_word_boxes(const float *__restrict__ p, 
         if ((threadIdx.x & 63) == 0)
             box[6 * (slot >> 6) + c] = c < 3 ? v[c] : -v[c];
     }
-    const float inv = 1.0f / (float)(1 << G.mshift);
-    const float x = -(v[3] + v[0]) * G.icx * inv, y = -(v[4] + v[1]) * G.icy * inv,
-                z = -(v[5] + v[2]) * G.icz * inv;
-    const float area = fmaxf(x * y, fmaxf(x * z, y * z));
-    if ((threadIdx.x & 63) == 0 && area <= BEAM_NARROW) {
+    float longest;
+    const float area = box_section(G, -(v[3] + v[0]), -(v[4] + v[1]), -(v[5] + v[2]), longest);
+    if ((threadIdx.x & 63) == 0 && area <= BEAM_NARROW * (float)(1 << (2 * G.mshift))) {
         atomicAdd(narrow, 1ull);
-        // pencil_sub's sub-blocks are at most 64
-        if (area <= BEAM_PENCIL * inv * inv && G.mshift >= 2 && G.mshift <= 4)
+        if (pencil_box(G, area, longest))
             atomicAdd(narrow + 1, 1ull);
     }
 }
 
-// The walk of a call, from its words: chosen = WALK_*.
+// The walk of a call, from its words: chosen = WALK_*.  Words that are no pencils are
+// walked one by one in the pencils' kernel, which has fewer wavefronts for that
+// (BEAM_WPC), so three words in four have to be (50,000 triangles in a volume, of 4,096
+// points 55, 70 and 85 % within a cell and the rest all over it: 5.50, 4.64 and 3.31 ms,
+// one by one 5.14, 4.53 and 3.48; 500,000: 8.73, 7.04 and 4.77, and 7.53, 6.19 and 4.51;
+// a terrain of 50,000: 2.36 and 1.73 at 70 and 85 %, and 2.26 and 1.84).
 __global__ void k_choose_walk(const unsigned long long *__restrict__ narrow, int64_t words, int any,
                               int beams, unsigned long long *__restrict__ chosen)
 {
     if (threadIdx.x == 0)
-        *chosen = any && 2 * (int64_t)narrow[1] >= words     ? WALK_PENCIL
+        *chosen = any && 4 * (int64_t)narrow[1] >= 3 * words ? WALK_PENCIL
                   : beams && 2 * (int64_t)narrow[0] >= words ? WALK_BEAM
                                                              : WALK_RAY;
 }
@@ -611,6 +612,7 @@ LEM_DEV int row_below(int x)
 // each word, how many there are; -1 if the rays walk one by one.  Sixteen slabs at a
 // time, a slab a lane: the arithmetic of one beam is the same in all its lanes, so four
 // words share its cost.
+template <bool PENCIL>
 LEM_DEV int beam_lists(const GridDev &G, const MacroTab &smq, const float *__restrict__ word_box,
                        int64_t w0, int64_t w1, float px, float py, float pz, bool from_p,
                        uint2 (*list)[BEAM_LIST])
@@ -621,6 +623,11 @@ LEM_DEV int beam_lists(const GridDev &G, const MacroTab &smq, const float *__res
     const float x0 = wb[0], y0 = wb[1], z0 = wb[2], x1 = wb[3], y1 = wb[4], z1 = wb[5];
     Beam b;
     bool ok = beam_of(G, px, py, pz, x0, y0, z0, x1, y1, z1, from_p, b);
+    if (PENCIL) {
+        float longest;
+        const float area = box_section(G, x1 - x0, y1 - y0, z1 - z0, longest);
+        ok &= pencil_box(G, area, longest);
+    }
     if (!ok)
         b.slabs = 0;
     int count = 0;
@@ -922,7 +929,7 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
         if constexpr (BEAM) {
             uint2 (*list)[BEAM_LIST] = s_list + (threadIdx.x >> 6) * BEAM_WORDS;
             for (int64_t word = w0; word < w1; word += BEAM_WORDS) {
-                const int cnt = beam_lists(G, smq, word_box, word, w1, P[0], P[1], P[2],
+                const int cnt = beam_lists<WALK == WALK_PENCIL>(G, smq, word_box, word, w1, P[0], P[1], P[2],
                                            SINK_MAJOR == REV, list);
                 __builtin_amdgcn_wave_barrier();
                 const int64_t left = w1 - word;

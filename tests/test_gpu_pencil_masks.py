@@ -72,3 +72,24 @@ def test_closest_hits_leave_out_pairs_of_one_row(native, scene, sink_major):
     assert np.array_equal(want, got.T if sink_major else got)
     assert np.array_equal(wd, gd.T if sink_major else gd)
     assert np.diag(want).sum() == 0
+
+
+@pytest.mark.parametrize("sink_major", [False, True])
+@pytest.mark.parametrize("narrow", [0.7, 0.8, 1.0])
+def test_wide_words_among_pencils(native, scene, narrow, sink_major):
+    """Points of one cluster and points all over the scene, on either side of the share
+    from which pencils are cast, and points along a line."""
+    tris, g, src, snk = scene
+    rng = np.random.default_rng(5)
+    side = tris.reshape(-1, 3).max()
+    n = int(narrow * 4096)
+    lanes = np.empty((4096, 3), np.float32)
+    lanes[:n] = rng.uniform(0, 0.2 * min(g.info.cell), (n, 3)) + [0.5 * side, 0.4 * side, 5.0]
+    lanes[n:] = rng.uniform([0, 0, -6], [side, side, 6], (4096 - n, 3))
+    line = np.linspace(0.1, 0.9, 4096)[:, None] * np.array([side, 0, 0]) + [0, 0.3 * side, 5.0]
+    for points in (lanes, line.astype(np.float32)):
+        a, b = (points, snk) if sink_major else (snk, points)
+        want = _mask(native.visibility_dense(a, b, tris)[0], len(b))
+        for from_sink in (False, True):
+            got = _mask(g.visibility(a, b, sink_major=sink_major, from_sink=from_sink)[0], len(points))
+            assert np.array_equal(want, got.T if sink_major else got)
