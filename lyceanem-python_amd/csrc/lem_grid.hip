@@ -550,51 +550,73 @@ constexpr int COUNTER_STRIDE = 512;  // uint64 elements
 constexpr int CLAIM_WORDS = 12;
 constexpr int CLAIM_DEPTH = 8;  // claims for each resident wavefront, before they are longer than a word
 
-// Box of the points of each word of 64 lane slots: box[word] = lo, hi; counts the
-// narrow ones, whose two longest sides span at most BEAM_NARROW square macro blocks
-// (narrow[0]), and the pencils (narrow[1]).  One wavefront a word.
-constexpr float BEAM_NARROW = 2.0f;
-__global__ __launch_bounds__(GB) void k_word_boxes(const float *__restrict__ p, int64_t n,
-                                                   const int32_t *__restrict__ order, GridDev G,
-                                                   float *__restrict__ box,
-                                                   unsigned long long *__restrict__ narrow)
-{
-    const int64_t slot = (int64_t)blockIdx.x * GB + threadIdx.x;
-    if ((slot & ~63ll) >= n)
-        return;  // wave-uniform
-    const int64_t at = slot < n ? slot : n - 1;  // lanes past the end repeat the last
-    const int64_t i = order ? (int64_t)order[at] : at;
-    float v[6] = {p[3 * i], p[3 * i + 1], p[3 * i + 2], -p[3 * i], -p[3 * i + 1], -p[3 * i + 2]};
-#pragma unroll
-    for (int c = 0; c < 6; ++c) {
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1)
-            v[c] = fminf(v[c], __shfl_xor(v[c], off));
-        if ((threadIdx.x & 63) == 0)
-            box[6 * (slot >> 6) + c] = c < 3 ? v[c] : -v[c];
-    }
-    float longest;
-    const float area = box_section(G, -(v[3] + v[0]), -(v[4] + v[1]), -(v[5] + v[2]), longest);
-    if ((threadIdx.x & 63) == 0 && area <= BEAM_NARROW * (float)(1 << (2 * G.mshift))) {
-        atomicAdd(narrow, 1ull);
-        if (pencil_box(G, area, longest))
-            atomicAdd(narrow + 1, 1ull);
-    }
-}
+// How the rays of a call walk: counts of its words, workgroups of k_word_boxes that are
+// done, and the walk (WALK_*).
+struct WalkPick {
+    unsigned long long narrow, pencil, done, walk;
+};
 
-// The walk of a call, from its words: chosen = WALK_*.  Words that are no pencils are
-// walked one by one in the pencils' kernel, which has fewer wavefronts for that
-// (BEAM_WPC), so three words in four have to be (50,000 triangles in a volume, of 4,096
-// points 55, 70 and 85 % within a cell and the rest all over it: 5.50, 4.64 and 3.31 ms,
-// one by one 5.14, 4.53 and 3.48; 500,000: 8.73, 7.04 and 4.77, and 7.53, 6.19 and 4.51;
-// a terrain of 50,000: 2.36 and 1.73 at 70 and 85 %, and 2.26 and 1.84).
-__global__ void k_choose_walk(const unsigned long long *__restrict__ narrow, int64_t words, int any,
-                              int beams, unsigned long long *__restrict__ chosen)
+// Box of the points of each word of 64 lane slots: box[word] = lo, hi.  A wavefront a
+// word.  Counts the narrow ones, whose two longest sides span at most BEAM_NARROW square
+// macro blocks, and the pencils; the last workgroup picks the walk.  Words that are no
+// pencils are walked one by one in the pencils' kernel, which has fewer wavefronts for
+// that (BEAM_WPC), so three words in four have to be (50,000 triangles in a volume, of
+// 4,096 points 55, 70 and 85 % within a cell and the rest all over it: 5.50, 4.64 and
+// 3.31 ms, one by one 5.14, 4.53 and 3.48; 500,000: 8.73, 7.04 and 4.77, and 7.53, 6.19
+// and 4.51; a terrain of 50,000: 2.36 and 1.73 at 70 and 85 %, and 2.26 and 1.84).
+// Bound by its atomics on the same words: a few for each of few large workgroups (2^20
+// points: 199 us with one or two a word, 14).
+constexpr float BEAM_NARROW = 2.0f;
+constexpr int BOXES_TB = 1024, BOXES_BLOCKS = 256;
+__global__ __launch_bounds__(BOXES_TB) void k_word_boxes(const float *__restrict__ p, int64_t n,
+                                                         const int32_t *__restrict__ order,
+                                                         GridDev G, int any, int beams,
+                                                         float *__restrict__ box, WalkPick *pick)
 {
-    if (threadIdx.x == 0)
-        *chosen = any && 4 * (int64_t)narrow[1] >= 3 * words ? WALK_PENCIL
-                  : beams && 2 * (int64_t)narrow[0] >= words ? WALK_BEAM
-                                                             : WALK_RAY;
+    __shared__ int s_n[2];
+    const int lane = threadIdx.x & 63;
+    if (threadIdx.x < 2)
+        s_n[threadIdx.x] = 0;
+    __syncthreads();
+    int n_narrow = 0, n_pencil = 0;
+    for (int64_t slot = (int64_t)blockIdx.x * BOXES_TB + threadIdx.x; (slot & ~63ll) < n;
+         slot += (int64_t)gridDim.x * BOXES_TB) {
+        const int64_t at = slot < n ? slot : n - 1;  // lanes past the end repeat the last
+        const int64_t i = order ? (int64_t)order[at] : at;
+        float v[6] = {p[3 * i], p[3 * i + 1], p[3 * i + 2], -p[3 * i], -p[3 * i + 1], -p[3 * i + 2]};
+#pragma unroll
+        for (int c = 0; c < 6; ++c) {
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1)
+                v[c] = fminf(v[c], __shfl_xor(v[c], off));
+            if (lane == 0)
+                box[6 * (slot >> 6) + c] = c < 3 ? v[c] : -v[c];
+        }
+        float longest;
+        const float area = box_section(G, -(v[3] + v[0]), -(v[4] + v[1]), -(v[5] + v[2]), longest);
+        const bool is_narrow = area <= BEAM_NARROW * (float)(1 << (2 * G.mshift));
+        n_narrow += is_narrow ? 1 : 0;
+        n_pencil += is_narrow && pencil_box(G, area, longest) ? 1 : 0;
+    }
+    if (lane == 0) {
+        atomicAdd(&s_n[0], n_narrow);
+        atomicAdd(&s_n[1], n_pencil);
+    }
+    __syncthreads();
+    if (threadIdx.x != 0)
+        return;
+    atomicAdd(&pick->narrow, (unsigned long long)s_n[0]);
+    atomicAdd(&pick->pencil, (unsigned long long)s_n[1]);
+    __threadfence();
+    if (atomicAdd(&pick->done, 1ull) + 1 == gridDim.x) {
+        const int64_t words = (n + 63) / 64;
+        __threadfence();
+        const int64_t narrow = (int64_t)atomicAdd(&pick->narrow, 0ull),
+                      pencil = (int64_t)atomicAdd(&pick->pencil, 0ull);
+        pick->walk = any && 4 * pencil >= 3 * words ? WALK_PENCIL
+                     : beams && 2 * narrow >= words ? WALK_BEAM
+                                                    : WALK_RAY;
+    }
 }
 
 constexpr int BEAM_WORDS = 4;  // words whose beams a wavefront finds at once, 16 lanes each
@@ -780,11 +802,11 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
     float *__restrict__ dist_out, unsigned long long *__restrict__ next_task, int skip_self,
     unsigned long long *__restrict__ par_count, uint2 *__restrict__ par_queue, int64_t par_cap,
     int perm, int claim, const int32_t *__restrict__ outer_order,
-    const float *__restrict__ word_box, const unsigned long long *__restrict__ chosen)
+    const float *__restrict__ word_box, const WalkPick *__restrict__ pick)
 {
     // every walk is launched that may serve, and the words' boxes decide
     constexpr bool BEAM = WALK != WALK_RAY;
-    if (chosen && (int)*chosen != WALK)
+    if (pick && (int)pick->walk != WALK)
         return;
     __shared__ uint2 s_list[BEAM ? GB / 64 * BEAM_WORDS : 1][BEAM_LIST];
     __shared__ uint32_t smqa[lds_table(WPC)];
@@ -944,14 +966,17 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
     }
 }
 
-// clears the 8 task counters of the persistent traversal and the two counts of narrow
-// words
-__global__ void k_zero_u64(unsigned long long *__restrict__ p)
+// clears the 8 task counters of the persistent traversal, the counts of its words and the
+// plane rays' count
+__global__ void k_zero_u64(unsigned long long *__restrict__ p, WalkPick *__restrict__ pick,
+                           unsigned long long *__restrict__ par_count)
 {
-    if (threadIdx.x < 9)
+    if (threadIdx.x < 8)
         p[threadIdx.x * COUNTER_STRIDE] = 0ull;
+    else if (threadIdx.x == 8)
+        *pick = WalkPick{0ull, 0ull, 0ull, WALK_RAY};
     else if (threadIdx.x == 9)
-        p[8 * COUNTER_STRIDE + 1] = 0ull;
+        *par_count = 0ull;
 }
 
 __global__ __launch_bounds__(GB) void k_zero_words(unsigned long long *__restrict__ p, int64_t n)
@@ -1121,7 +1146,7 @@ struct VisWs {
 
 constexpr int MORTON_BITS = 30;
 // workspace head: the 8 task counters (4 KB apart), then the point bounds (afterwards
-// the count of narrow words)
+// the walk's pick)
 constexpr int64_t VIS_HEAD = 8 * 8 * COUNTER_STRIDE + 256;
 
 inline int64_t vis_sort_bytes(int64_t n)
@@ -1627,7 +1652,14 @@ extern "C" int lem_visibility_grid(const float *src, int64_t S, const float *snk
         // 65,536 words: 6.0 -> 2.0).
         const int claim =
             (int)std::max<int64_t>(1, std::min<int64_t>(CLAIM_WORDS, words / (nwg * 4 * CLAIM_DEPTH)));
-        hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, L.counter);
+        // queue of the rays along grid planes, walked afterwards by
+        // k_visibility_grid_par over as many workgroups as fill the chip
+        char *qb = reinterpret_cast<char *>(workspace) + (need - PAR_QUEUE_BYTES);
+        unsigned long long *pcount = reinterpret_cast<unsigned long long *>(qb);
+        uint2 *pq = reinterpret_cast<uint2 *>(qb + 256);
+        // the walk's pick takes the place of the point bounds
+        WalkPick *pk = reinterpret_cast<WalkPick *>(L.counter + 8 * COUNTER_STRIDE);
+        hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, L.counter, pk, pcount);
         // Beams and pencils serve rays in a spatial order whose words are narrow.
         // Pencils, any hit: 5,000 and 50,000 triangles, 3,600 sources within a tenth of
         // a cell x 30,000 sinks, 5.25 and 9.95 ms one by one -> 2.85 and 6.66 (from the
@@ -1641,29 +1673,24 @@ extern "C" int lem_visibility_grid(const float *src, int64_t S, const float *snk
         // word: 2.56 and 7.45 -> 2.91 and 8.65.  Below 2^18 rays the boxes and the
         // launches are not worth it.  The boxes take the place of the Morton keys.
         float *word_box = nullptr;
-        unsigned long long *chosen = nullptr;
-        if (order && semantics != LEM_SEM_NATIVE && (double)S * (double)K >= 262144.0) {
+        const WalkPick *pick = nullptr;
+        const bool beams = sink_major && !rev, pencils = any && G.mshift >= 2 && G.mshift <= 4;
+        if (order && semantics != LEM_SEM_NATIVE && (beams || pencils) &&
+            (double)S * (double)K >= 262144.0) {
             word_box = reinterpret_cast<float *>(L.k0);
-            unsigned long long *narrow = L.counter + 8 * COUNTER_STRIDE;
-            chosen = narrow + 2;
-            hipLaunchKernelGGL(k_word_boxes, dim3((unsigned)nbl), dim3(GB), 0, st,
-                               sink_major ? src : snk, NI, order, G, word_box, narrow);
-            hipLaunchKernelGGL(k_choose_walk, dim3(1), dim3(64), 0, st, narrow, Wn, any ? 1 : 0,
-                               sink_major && !rev ? 1 : 0, chosen);
+            pick = pk;
+            hipLaunchKernelGGL(k_word_boxes,
+                               dim3((unsigned)std::min<int64_t>(ceil_div(NI, BOXES_TB), BOXES_BLOCKS)),
+                               dim3(BOXES_TB), 0, st, sink_major ? src : snk, NI, order, G,
+                               any ? 1 : 0, beams ? 1 : 0, word_box, pk);
         }
         const int64_t nbeam =
             std::max<int64_t>(1, std::min<int64_t>(ceil_div(words, 4), (int64_t)cus * BEAM_WPC));
-        // queue of the rays along grid planes, walked afterwards by
-        // k_visibility_grid_par over as many workgroups as fill the chip
-        char *qb = reinterpret_cast<char *>(workspace) + (need - PAR_QUEUE_BYTES);
-        unsigned long long *pcount = reinterpret_cast<unsigned long long *>(qb);
-        uint2 *pq = reinterpret_cast<uint2 *>(qb + 256);
-        hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(GB), 0, st, pcount, 1);
 #define LEM_WALK(A, M, SM, R, WP, WALK, NWG)                                                  \
     hipLaunchKernelGGL((k_visibility_grid_lds<A, M, SM, R, WP, WALK>), dim3((unsigned)(NWG)), \
                        dim3(GB), 0, st, src, S, snk, K, G, cell_start, rc4, bx4, mq,          \
                        info->nmacro, order, hb, dist, L.counter, skip_self, pcount, pq,       \
-                       PAR_QUEUE_CAP, perm ? 1 : 0, claim, outer_order, word_box, chosen)
+                       PAR_QUEUE_CAP, perm ? 1 : 0, claim, outer_order, word_box, pick)
 #define LEM_VGL(A, M, SM, R, WP)                                                              \
     do {                                                                                      \
         if constexpr (A && SM == LEM_SEM_NUMBA)                                               \
