@@ -206,16 +206,22 @@ LEM_DEV float box_section(const GridDev &G, float dx, float dy, float dz, float 
 }
 
 // Whether the rays to the points of a box are a pencil.  The points of a line span a fan
-// of cells, not one: at most a block of 4 x 4 x 4 cells, and one cell where blocks are
-// larger (as pencils and one by one, from the line's end: 5,000 triangles in a volume,
-// 4 cells a word, 353 and 491 us; 150,000, 4 cells, 709 and 702; 500,000 in blocks of 8
-// cells, 1, 2 and 4 cells, 1.06 and 1.04, 1.40 and 1.26, 2.05 and 1.61 ms).  Blocks
-// have at most 64 sub-blocks, a lane each.
+// of cells, not one, and the wider it is the fewer of its rays come near a triangle:
+// at most 8 cells, half as many in a full grid, and half or a quarter of that where
+// blocks are larger than 4 x 4 x 4 cells.  As pencils and one by one, us, from a line of
+// 1,024 points (8 cells: 256) to 4,000, cells a word:
+//                                1            2            4            8
+//   volume of 5,000, blocks of 4   324, 445     326, 467     353, 491     301, 357
+//   50,000 (full)                  623, 762     776, 896   1,045, 1,124   578, 579
+//   150,000 (full)               1,069, 1,101 1,369, 1,372 1,853, 1,791   854, 822
+//   500,000 (full), blocks of 8  1,049, 1,036 1,399, 1,269 2,055, 1,590 1,252, 797
+//   terrain of 10^6, blocks of 8   336, 406     333, 433     382, 456     383, 379
+// Blocks have at most 64 sub-blocks, a lane each.
 constexpr float PENCIL_SECTION = 0.25f;
-LEM_DEV bool pencil_box(const GridDev &G, float section, float longest)
+LEM_DEV bool pencil_box(const GridDev &G, float section, float longest, bool full)
 {
-    return (section <= PENCIL_SECTION) & (longest <= (G.mshift == 2 ? 4.0f : 1.0f)) &
-           (G.mshift >= 2) & (G.mshift <= 4);
+    const float bound = G.mshift == 2 ? (full ? 4.0f : 8.0f) : (full ? 1.0f : 4.0f);
+    return (section <= PENCIL_SECTION) & (longest <= bound) & (G.mshift >= 2) & (G.mshift <= 4);
 }
 
 // Sub-block s of block (jx, jy, jz): its first cell, and whether the beam meets it.

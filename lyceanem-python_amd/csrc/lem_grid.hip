@@ -551,22 +551,36 @@ constexpr int CLAIM_WORDS = 12;
 constexpr int CLAIM_DEPTH = 8;  // claims for each resident wavefront, before they are longer than a word
 
 // How the rays of a call walk: counts of its words, workgroups of k_word_boxes that are
-// done, and the walk (WALK_*).
+// done, the walk (WALK_*), and whether the grid is full: several triangles to a cell,
+// and content that fills the macro blocks.
 struct WalkPick {
-    unsigned long long narrow, pencil, done, walk;
+    unsigned long long narrow, pencil, done, walk, full;
 };
 
 // Box of the points of each word of 64 lane slots: box[word] = lo, hi.  A wavefront a
 // word.  Counts the narrow ones, whose two longest sides span at most BEAM_NARROW square
-// macro blocks, and the pencils; the last workgroup picks the walk.  Words that are no
-// pencils are walked one by one in the pencils' kernel, which has fewer wavefronts for
-// that (BEAM_WPC), so three words in four have to be (50,000 triangles in a volume, of
-// 4,096 points 55, 70 and 85 % within a cell and the rest all over it: 5.50, 4.64 and
-// 3.31 ms, one by one 5.14, 4.53 and 3.48; 500,000: 8.73, 7.04 and 4.77, and 7.53, 6.19
-// and 4.51; a terrain of 50,000: 2.36 and 1.73 at 70 and 85 %, and 2.26 and 1.84).
+// macro blocks, and the pencils; the last workgroup picks the walk.
+//
+// Words that are no pencils are walked one by one in the pencils' kernel, which has fewer
+// wavefronts for that (BEAM_WPC): half of the words have to be pencils, three in four in
+// a full grid of blocks larger than 4 x 4 x 4 cells.  4,096 points of which 55, 70 and 85
+// % lie within a cell and the rest all over the scene, x 4,000: among 50,000 triangles
+// 5.50, 4.64 and 3.31 ms, one by one 5.14, 4.53 and 3.48; among 500,000 (full, blocks of
+// 8) 8.73, 7.04 and 4.77, and 7.53, 6.19 and 4.51; over a terrain of 50,000, 2.36 and 1.73
+// at 70 and 85 %, and 2.26 and 1.84.  In clusters of 64, which share many words, 50,000
+// triangles: 2.16 and 2.52.
+//
+// Beams skip what is empty for a word at a time, but a list goes on behind its rays'
+// hits: they lose in full grids, where rays end early.  As beams and one by one, closest
+// hit of 16,384 points x 2,000 in a volume of 5,000, 50,000, 150,000 and 500,000
+// triangles (1.0, 1.5, 2.2 and 3.5 to a cell, content 0.95 to 0.85), words of a quarter
+// square block: 3.39, 10.04, 16.9 and 24.3 ms, and 3.96, 9.78, 15.8 and 22.0; over
+// terrains of 5,000 to 10^6 (2.5 to 1.5, content 0.35 to 0.06): 2.24, 2.78, 2.92 and
+// 1.74, and 2.50, 3.53, 3.45 and 2.53.
+//
 // Bound by its atomics on the same words: a few for each of few large workgroups (2^20
 // points: 199 us with one or two a word, 14).
-constexpr float BEAM_NARROW = 2.0f;
+constexpr float BEAM_NARROW = 2.0f, BEAM_FULL = 0.6f;
 constexpr int BOXES_TB = 1024, BOXES_BLOCKS = 256;
 __global__ __launch_bounds__(BOXES_TB) void k_word_boxes(const float *__restrict__ p, int64_t n,
                                                          const int32_t *__restrict__ order,
@@ -574,6 +588,7 @@ __global__ __launch_bounds__(BOXES_TB) void k_word_boxes(const float *__restrict
                                                          float *__restrict__ box, WalkPick *pick)
 {
     __shared__ int s_n[2];
+    const bool full = pick->full != 0;
     const int lane = threadIdx.x & 63;
     if (threadIdx.x < 2)
         s_n[threadIdx.x] = 0;
@@ -596,7 +611,7 @@ __global__ __launch_bounds__(BOXES_TB) void k_word_boxes(const float *__restrict
         const float area = box_section(G, -(v[3] + v[0]), -(v[4] + v[1]), -(v[5] + v[2]), longest);
         const bool is_narrow = area <= BEAM_NARROW * (float)(1 << (2 * G.mshift));
         n_narrow += is_narrow ? 1 : 0;
-        n_pencil += is_narrow && pencil_box(G, area, longest) ? 1 : 0;
+        n_pencil += is_narrow && pencil_box(G, area, longest, full) ? 1 : 0;
     }
     if (lane == 0) {
         atomicAdd(&s_n[0], n_narrow);
@@ -608,15 +623,17 @@ __global__ __launch_bounds__(BOXES_TB) void k_word_boxes(const float *__restrict
     atomicAdd(&pick->narrow, (unsigned long long)s_n[0]);
     atomicAdd(&pick->pencil, (unsigned long long)s_n[1]);
     __threadfence();
-    if (atomicAdd(&pick->done, 1ull) + 1 == gridDim.x) {
-        const int64_t words = (n + 63) / 64;
-        __threadfence();
-        const int64_t narrow = (int64_t)atomicAdd(&pick->narrow, 0ull),
-                      pencil = (int64_t)atomicAdd(&pick->pencil, 0ull);
-        pick->walk = any && 4 * pencil >= 3 * words ? WALK_PENCIL
-                     : beams && 2 * narrow >= words ? WALK_BEAM
-                                                    : WALK_RAY;
-    }
+    if (atomicAdd(&pick->done, 1ull) + 1 != gridDim.x)
+        return;
+    __threadfence();
+    const int64_t words = (n + 63) / 64;
+    const int64_t narrow = (int64_t)atomicAdd(&pick->narrow, 0ull),
+                  pencil = (int64_t)atomicAdd(&pick->pencil, 0ull);
+    const bool pencils =
+        any && (full && G.mshift != 2 ? 4 * pencil >= 3 * words : 2 * pencil >= words);
+    pick->walk = pencils                                 ? WALK_PENCIL
+                 : beams && !full && 2 * narrow >= words ? WALK_BEAM
+                                                         : WALK_RAY;
 }
 
 constexpr int BEAM_WORDS = 4;  // words whose beams a wavefront finds at once, 16 lanes each
@@ -637,7 +654,7 @@ LEM_DEV int row_below(int x)
 template <bool PENCIL>
 LEM_DEV int beam_lists(const GridDev &G, const MacroTab &smq, const float *__restrict__ word_box,
                        int64_t w0, int64_t w1, float px, float py, float pz, bool from_p,
-                       uint2 (*list)[BEAM_LIST])
+                       bool full, uint2 (*list)[BEAM_LIST])
 {
     const int lane = threadIdx.x & 63, q = lane >> 4, l = lane & 15;
     const int64_t w = w0 + q < w1 ? w0 + q : w1 - 1;
@@ -648,7 +665,7 @@ LEM_DEV int beam_lists(const GridDev &G, const MacroTab &smq, const float *__res
     if (PENCIL) {
         float longest;
         const float area = box_section(G, x1 - x0, y1 - y0, z1 - z0, longest);
-        ok &= pencil_box(G, area, longest);
+        ok &= pencil_box(G, area, longest, full);
     }
     if (!ok)
         b.slabs = 0;
@@ -950,9 +967,10 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
         };
         if constexpr (BEAM) {
             uint2 (*list)[BEAM_LIST] = s_list + (threadIdx.x >> 6) * BEAM_WORDS;
+            const bool full = pick && pick->full != 0;
             for (int64_t word = w0; word < w1; word += BEAM_WORDS) {
-                const int cnt = beam_lists<WALK == WALK_PENCIL>(G, smq, word_box, word, w1, P[0], P[1], P[2],
-                                           SINK_MAJOR == REV, list);
+                const int cnt = beam_lists<WALK == WALK_PENCIL>(
+                    G, smq, word_box, word, w1, P[0], P[1], P[2], SINK_MAJOR == REV, full, list);
                 __builtin_amdgcn_wave_barrier();
                 const int64_t left = w1 - word;
                 for (int q = 0; q < BEAM_WORDS && q < left; ++q)
@@ -966,17 +984,40 @@ __global__ __launch_bounds__(GB, WPC) void k_visibility_grid_lds(
     }
 }
 
-// clears the 8 task counters of the persistent traversal, the counts of its words and the
-// plane rays' count
-__global__ void k_zero_u64(unsigned long long *__restrict__ p, WalkPick *__restrict__ pick,
-                           unsigned long long *__restrict__ par_count)
+// Clears the 8 task counters of the persistent traversal, the counts of its words and the
+// plane rays' count, and says whether the grid is full (nmacro: blocks to look at, 0
+// where cells hold few triangles).  One workgroup.
+constexpr int START_TB = 1024;
+__global__ __launch_bounds__(START_TB) void k_start_walk(unsigned long long *__restrict__ p,
+                                                         WalkPick *__restrict__ pick,
+                                                         unsigned long long *__restrict__ par_count,
+                                                         const uint2 *__restrict__ mq, int nmacro)
 {
+    __shared__ float s_content[START_TB / 64];
     if (threadIdx.x < 8)
         p[threadIdx.x * COUNTER_STRIDE] = 0ull;
     else if (threadIdx.x == 8)
-        *pick = WalkPick{0ull, 0ull, 0ull, WALK_RAY};
-    else if (threadIdx.x == 9)
         *par_count = 0ull;
+    float content = 0.0f;  // of the blocks, as a fraction of each
+    for (int m = threadIdx.x; m < nmacro; m += START_TB) {
+        const uint2 q = mq[m];
+        const int x = (int)(q.x >> 24) - (int)(q.x & 255u),
+                  y = (int)(q.y & 255u) - (int)((q.x >> 8) & 255u),
+                  z = (int)((q.y >> 8) & 255u) - (int)((q.x >> 16) & 255u);
+        content += (float)max(x, 0) * (float)max(y, 0) * (float)max(z, 0) * (1.0f / (255 * 255 * 255));
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+        content += __shfl_xor(content, off);
+    if ((threadIdx.x & 63) == 0)
+        s_content[threadIdx.x >> 6] = content;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < START_TB / 64; ++w)
+            content += s_content[w];
+        const bool full = content > BEAM_FULL * (float)nmacro;
+        *pick = WalkPick{0ull, 0ull, 0ull, WALK_RAY, full ? 1ull : 0ull};
+    }
 }
 
 __global__ __launch_bounds__(GB) void k_zero_words(unsigned long long *__restrict__ p, int64_t n)
@@ -1659,7 +1700,8 @@ extern "C" int lem_visibility_grid(const float *src, int64_t S, const float *snk
         uint2 *pq = reinterpret_cast<uint2 *>(qb + 256);
         // the walk's pick takes the place of the point bounds
         WalkPick *pk = reinterpret_cast<WalkPick *>(L.counter + 8 * COUNTER_STRIDE);
-        hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, L.counter, pk, pcount);
+        hipLaunchKernelGGL(k_start_walk, dim3(1), dim3(START_TB), 0, st, L.counter, pk, pcount, mq,
+                           2 * info->nrefs > 3 * info->ncells ? info->nmacro : 0);
         // Beams and pencils serve rays in a spatial order whose words are narrow.
         // Pencils, any hit: 5,000 and 50,000 triangles, 3,600 sources within a tenth of
         // a cell x 30,000 sinks, 5.25 and 9.95 ms one by one -> 2.85 and 6.66 (from the
