@@ -60,7 +60,7 @@ struct GwPair {
 
 template <bool LOSSY>
 LEM_DEV GwPair gw_pair(float xs, float ys, float zs, double xk, double yk, double zk, float nx,
-                       float ny, float nz, float ex, float ey, float ez, double kw, float alpha)
+                       float ny, float nz, float ex, float ey, float ez, double kw, double alpha)
 {
 #pragma clang fp contract(fast)
     const float FRONT = -0.15915494309189535f;
@@ -71,9 +71,9 @@ LEM_DEV GwPair gw_pair(float xs, float ys, float zs, double xk, double yk, doubl
     const float cs = ux * nx + uy * ny + uz * nz;
     float amp = ir;
     if (LOSSY)
-        amp *= expf(-alpha * (float)p.r);
+        amp *= expf((float)(-alpha * p.r));  // rounded once: alpha r may be large
     const float Gr = amp * p.c, Gi = amp * p.s;
-    const float ar = -alpha - ir, ai = -(float)kw;
+    const float ar = -(float)alpha - ir, ai = -(float)kw;
     const float f_ = FRONT * cs;
     const float ue = ux * ex + uy * ey + uz * ez;
     GwPair g;
@@ -158,7 +158,7 @@ LEM_DEV bf16x8 flipped(const bf16x8 &x)
 template <bool LOSSY>
 LEM_DEV void gw_finish(f32x16 (&re)[3], f32x16 (&im)[3], const float *__restrict__ src, int64_t S,
                        const float *__restrict__ snk, const float *__restrict__ snk_n, int64_t K,
-                       int64_t k0, float ex, float ey, float ez, double kw, float alpha,
+                       int64_t k0, float ex, float ey, float ez, double kw, double alpha,
                        const float2 *__restrict__ Wf, float2 *__restrict__ out, int col, int64_t f)
 {
     const int lane = threadIdx.x & 63, half = lane >> 5;
@@ -215,7 +215,7 @@ template <bool LOSSY>
 __global__ __launch_bounds__(512, 2) void k_gw_tile(
     const float *__restrict__ src, int64_t S, const float *__restrict__ snk,
     const float *__restrict__ snk_n, int64_t K, float ex, float ey, float ez,
-    const double *__restrict__ kf, float alpha, const float2 *__restrict__ W,
+    const double *__restrict__ kf, double alpha, const float2 *__restrict__ W,
     float2 *__restrict__ out)
 {
     // [buffer][plane][half-wave's k][row or set] x 8 bfloat16
@@ -360,7 +360,7 @@ template <bool LOSSY>
 __global__ __launch_bounds__(64 * GW_MAX_WAVES, 2) void k_gw_mfma(
     const float *__restrict__ src, int64_t S, const float *__restrict__ snk,
     const float *__restrict__ snk_n, int64_t K, float ex, float ey, float ez,
-    const double *__restrict__ kf, float alpha, const float2 *__restrict__ W,
+    const double *__restrict__ kf, double alpha, const float2 *__restrict__ W,
     float2 *__restrict__ out)
 {
     extern __shared__ float s_part[];  // nw / 2 wavefronts' sums
@@ -506,10 +506,10 @@ extern "C" int lem_gw_mfma(const float *src, int64_t S, float pol_x, float pol_y
         dim3 grid((unsigned)ceil_div(K, TILE), (unsigned)F);                                  \
         if (alpha != 0.0)                                                                     \
             hipLaunchKernelGGL(KERNEL<true>, grid, dim3(THREADS), LDS, st, src, S, snk, snk_n, K, \
-                               pol_x, pol_y, pol_z, wavenumbers, (float)alpha, W2, out2);     \
+                               pol_x, pol_y, pol_z, wavenumbers, alpha, W2, out2);     \
         else                                                                                  \
             hipLaunchKernelGGL(KERNEL<false>, grid, dim3(THREADS), LDS, st, src, S, snk, snk_n, K, \
-                               pol_x, pol_y, pol_z, wavenumbers, (float)alpha, W2, out2);     \
+                               pol_x, pol_y, pol_z, wavenumbers, alpha, W2, out2);     \
     } while (0)
     if (nw)
         LEM_GW(k_gw_mfma, GW_M / 2, 64 * nw, nw / 2 * 96 * 64 * 4);
