@@ -151,8 +151,9 @@ class C1:
             "kernel_ms": vis,
             "roofline": {"bound": "valu", "achieved": achieved / 1e12, "peak": PEAK_FP32 / 1e12,
                          "unit": "TFLOP/s", "frac": achieved / PEAK_FP32, "traffic": None,
-                         "basis": "the linear tests of every ray x triangle (the Moller-Trumbore "
-                                  "predicate follows only where they pass)"},
+                         "basis": "work answered, not instructions issued: 20 FP32 flops of linear "
+                                  "tests for every ray x triangle, those that a wavefront's box of "
+                                  "directions spares it included"},
             "extra": {"field_kernel_ms": fld,
                       "field_gpairs_per_s": self.rays() / (fld * 1e-3) / 1e9,
                       "mt_tests": self.rays() * self.T},
@@ -285,7 +286,7 @@ class C2:
                                   "triangle reference of every crossed cell)",
                          "achieved_executed": executed / 1e12,
                          "frac_executed": executed / PEAK_FP32,
-                         "basis_executed": "46 FP32 flops x the MT tests the kernel performs",
+                         "basis_executed": "46 FP32 flops x the MT tests of the one-by-one walk",
                          "traffic": traffic,
                          "traffic_source": None if traffic is None else
                          "profiles/" + os.path.basename(TRAFFIC_PROFILE) + " (bytes per ray x "
@@ -475,7 +476,7 @@ class C3:
                                   "front-to-back DDA performs up to the first hit",
                          "achieved_executed": executed / 1e12,
                          "frac_executed": executed / PEAK_FP32,
-                         "basis_executed": "46 FP32 flops x the MT tests the kernel performs",
+                         "basis_executed": "46 FP32 flops x the MT tests of the one-by-one walk",
                          "traffic": None},
             "extra": {"gpairs_per_s": self.rays() / ((vis + rest) * 1e-3) / 1e9,
                       "leg1_walk": "from scatterer" if self.from_sink else "from array",

@@ -579,7 +579,7 @@ struct WalkPick {
 // 1.74, and 2.50, 3.53, 3.45 and 2.53.
 //
 // Bound by its atomics on the same words: a few for each of few large workgroups (2^20
-// points: 199 us with one or two a word, 14).
+// points: 199 us with one or two a word, 14 to 23).
 constexpr float BEAM_NARROW = 2.0f, BEAM_FULL = 0.6f;
 constexpr int BOXES_TB = 1024, BOXES_BLOCKS = 256;
 __global__ __launch_bounds__(BOXES_TB) void k_word_boxes(const float *__restrict__ p, int64_t n,
@@ -707,10 +707,10 @@ LEM_DEV int beam_lists(const GridDev &G, const MacroTab &smq, const float *__res
 // The wavefront's rays through the n blocks of its word's list.
 //
 // A terrain of 10^6 triangles, 1,024 x 1,024 sources 30 m up, 512 sinks, closest hit:
-// 37.1 ms one by one, 3,320 vector instructions a word of 64 rays; 21.6 ms as beams,
-// 1,370 of them (290 for the lists).  What bounds it now is the gather of cell boxes
-// and triangles: the address units are busy 65 % of the time, with 56 loads a word
-// (77 one by one).  (Measured and left: the next cell's box loaded before this one's
+// 37.1 ms one by one, 3,320 vector instructions a word of 64 rays; 21.0 ms as beams,
+// 1,390 of them (290 for the lists).  What bounds it now is the chain of cell box and
+// triangles, 58 loads a word (77 one by one): four waves a SIMD wait half of their time,
+// the address units are busy 58 % of it and the vector units 45 %.  (Measured and left: the next cell's box loaded before this one's
 // triangles are tested, the same; one word's beam at a time over 64 lanes, 26.1 ms.)
 template <bool ANY, int SEM>
 LEM_DEV bool beam_cast(bool walk, const Ray &r, const Ray &rt, const GridDev &G,

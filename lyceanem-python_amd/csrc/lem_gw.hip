@@ -28,8 +28,8 @@
 // sets x 3 components, and preparing it takes about 500 vector instructions: what
 // bounds both kernels below is that the two only overlap between wavefronts of a
 // SIMD, of which the 96 sums and 48 partial ones leave room for two.  64 x 64
-// sources, 16,384 sinks, 16 frequencies: 13.87 ms (FP32 instructions) -> 8.78 ms;
-// 32 x 32 sources, 2,720 sinks, one frequency: 186 -> 73 us.  (Measured and
+// sources, 16,384 sinks, 16 frequencies: 13.85 ms (FP32 instructions) -> 8.77 ms;
+// 32 x 32 sources, 2,720 sinks, one frequency: 188 -> 73 us.  (Measured and
 // left: pairs of wavefronts that share G in LDS, 9.3 ms and 98 us; matrix and vector
 // instructions interleaved in one wavefront, 12 ms and more, with registers spilled;
 // all six products in one chain, 8.48 ms and 74 us with an error of 3.4e-8.)
@@ -461,9 +461,9 @@ __global__ __launch_bounds__(64 * GW_MAX_WAVES, 2) void k_gw_mfma(
 // units of 0.1 us: a step of k_gw_tile's workgroup, one a CU, 21; a step of a
 // k_gw_mfma wavefront 38 alone on its SIMD, 52 beside a second one; adding the
 // sums about two steps a level.  Measured (k_gw_tile / k_gw_mfma, us): 1,024
-// sources x 2,720 sinks 136 / 78, 4,096 x 2,720 440 / 197, 2,304 x 5,600 x 3
-// frequencies 580 / 536; 4,096 x 16,384 545 / 719, 4,096 x 11,328 x 3 1,465 / 1,559,
-// 4,096 x 16,384 x 16 8,383 / 11,137.
+// sources x 2,720 sinks 134 / 74, 4,096 x 2,720 447 / 199, 2,304 x 5,600 x 3
+// frequencies 592 / 524; 4,096 x 16,384 593 / 755, 4,096 x 11,328 x 3 1,591 / 1,622,
+// 4,096 x 16,384 x 16 9,038 / 11,357.
 inline int gw_waves(int64_t K, int64_t F, int64_t steps)
 {
     const int64_t tiles = K / GW_M * 2 * F;
